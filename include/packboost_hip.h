@@ -314,6 +314,16 @@ int pb_set_bin_layout(pb_ctx* ctx, int32_t layout);
 int pb_pack_bins4(const uint8_t* bins_dev, int64_t n, int64_t ld, int32_t F, uint8_t* out_dev,
                   void* stream);
 
+/* The frontier kernels' feature-major bins from row-major ones (booster.py:419-426's
+ * bins.t().contiguous()): out_dev[f][r] = src_dev[(perm_dev ? perm_dev[r] : r) * row_stride + f]
+ * for r < n, 0 for rows n .. n_out-1. src_dev: one byte per code, any alignment; perm_dev: optional
+ * int64 [n] row gather (e.g. the era-major order, every entry a row of src). limit > 0:
+ * over_dev[0] |= 1 if any moved code is >= limit (the caller clears it). n <= n_out <= ld,
+ * n_out % 16 == ld % 16 == 0; out_dev 16-byte aligned. */
+int pb_transpose_bins(const uint8_t* src_dev, int64_t n, int64_t row_stride, int32_t F, const int64_t* perm_dev,
+                      uint8_t* out_dev, int64_t n_out, int64_t ld, int32_t limit, int32_t* over_dev,
+                      void* stream);
+
 /* apply_bins (data.py:93-111): bins[f][r] = min(searchsorted(edges[:, f], x, side="left"),
  * max_bins - 1) with NumPy's NaN-last order, x = xt[f][perm ? perm[r] : r] (xt: float32
  * [F][ld_x] column-major values; perm: optional int64 [n] row gather, e.g. the era-major

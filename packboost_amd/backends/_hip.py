@@ -36,7 +36,7 @@ EXPORTED_SYMBOLS = (
     "pb_forest_create", "pb_forest_predict", "pb_forest_destroy", "pb_pack_bins4",
     "pb_set_bin_layout", "pb_select_subsets", "pb_rowlist_work_elems", "pb_rowlist_partition",
     "pb_rowlist_gather", "pb_best_thresholds", "pb_pick_sequential", "pb_set_segment_mode", "pb_rowlist_noalloc_max_segments",
-    "pb_rowlist_partition_noalloc",
+    "pb_rowlist_partition_noalloc", "pb_transpose_bins",
 )
 
 
@@ -117,6 +117,7 @@ _SIGNATURES = {
     "pb_forest_destroy": (ctypes.c_int, [_VP]),
     "pb_quantile_edges": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _VP, _I32, _VP]),
     "pb_apply_bins": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _I32, _I32, _VP, _VP, _I64, _VP]),
+    "pb_transpose_bins": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _VP, _I64, _I64, _I32, _VP, _VP]),
     "pb_pack_bins4": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _VP]),
     "pb_set_bin_layout": (ctypes.c_int, [_VP, _I32]),
     "pb_select_subsets": (ctypes.c_int, [_VP, _VP, _I32, _I32, _VP, _VP]),

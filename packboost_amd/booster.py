@@ -29,7 +29,7 @@ from .data import (BinningResult, apply_bins, apply_bins_device, detect_prebinne
                    era_major_order, feature_names_or_default, preprocess_features,
                    quantile_bin_device)
 from .engine import (DeviceFit, column_major_bins, depth_log_from_round, padded_rows,
-                     subset_size, tree_arrays_from_log)
+                     subset_size, transpose_rows, tree_arrays_from_log)
 
 
 # ------------------------------------------------------------------ tree structures
@@ -129,9 +129,11 @@ def _to_column_major(bins, device: torch.device) -> torch.Tensor:
     if t.dtype not in (torch.uint8, torch.int8):
         t = t.to(torch.uint8)
     N, F = t.shape
-    ld = padded_rows(int(N))
-    out = torch.zeros((int(F), ld), dtype=torch.uint8, device=device)
-    out[:, :N] = t.to(device).view(torch.uint8).t()
+    out = torch.empty((int(F), padded_rows(int(N))), dtype=torch.uint8, device=device)
+    t = t.to(device).view(torch.uint8)
+    if not transpose_rows(t, out):
+        out[:, :N] = t.t()
+        out[:, N:] = 0
     return out
 
 
@@ -273,17 +275,17 @@ class PackBoost:
             "cuda", torch.cuda.current_device())
         if isinstance(X, torch.Tensor) and not X.dtype.is_floating_point:
             self._binner = BinningResult(bins=np.empty((0, F), np.uint8), bin_edges=None, prebinned=True)
-            bins_fm = column_major_bins(X, perm, device)
+            bins_fm = column_major_bins(X, perm, device, limit=cfg.max_bins)
         elif not isinstance(X, torch.Tensor) and (bool(cfg.prebinned) or detect_prebinned(X_arr, cfg.max_bins)):
             self._binner = preprocess_features(X_arr, cfg.max_bins, assume_prebinned=bool(cfg.prebinned))
-            bins_fm = column_major_bins(self._binner.bins, perm, device)
+            bins_fm = column_major_bins(self._binner.bins, perm, device, limit=cfg.max_bins)
         else:
             # quantile binning on the device, rows gathered era-major (data.py:44-56)
             bins_fm, edges = quantile_bin_device(X if isinstance(X, torch.Tensor) else X_arr,
                                                  cfg.max_bins, device, perm=perm)
             self._binner = BinningResult(bins=np.empty((0, F), np.uint8), bin_edges=edges,
                                          prebinned=False)
-        if N and int(bins_fm[:, :N].max().item()) >= cfg.max_bins:
+        if N and cfg.max_bins <= 0:
             raise ValueError("bins must lie in [0, max_bins)")
         y_dev = torch.from_numpy(y_np if perm is None else y_np[perm]).to(device)
         self._perm = perm

@@ -113,7 +113,126 @@ __global__ __launch_bounds__(kBlock) void pack_bins4_kernel(const uint8_t* __res
     }
 }
 
+// Row-major bin codes [n][F] (row stride `stride` bytes, any alignment) to the histogram's
+// column-major [F][ld], optionally gathering rows through a permutation; rows n .. n_out-1 become 0.
+// Bound by HBM (every byte read and written once). A workgroup moves a tile of 256 rows x 128
+// features: each thread reads 16 features of 4 consecutive rows (8 lanes cover 128 contiguous
+// bytes of a row), transposes them as 4x4 bytes in registers and puts one dword (4 rows) per
+// feature into LDS, whose odd row stride spreads the 8 lanes of a row over the banks; the tile then
+// leaves as 16-byte stores, 256 contiguous bytes per column. Feature tiles are the fastest grid
+// dimension, so the workgroups in flight read whole rows. 2.4M x 2376 codes take 2.34 ms (4.9 TB/s,
+// this card's copy rate; 4.65 ms with the loads behind per-row guards, 28 ms as torch's strided
+// copy), 2.72 ms through a random row permutation.
+// limit > 0: *over is set when some code is >= limit (codes compared four at a time).
+constexpr int kTrRows = 256;
+constexpr int kTrFeats = 128;
+
+struct __attribute__((packed)) Bytes16 {
+    uint32_t w[4];
+};
+
+__device__ __forceinline__ void transpose4x4_bytes(const uint32_t (&r)[4], uint32_t (&c)[4]) {
+    const uint32_t ab0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);  // a0 b0 a1 b1
+    const uint32_t ab1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);  // a2 b2 a3 b3
+    const uint32_t cd0 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
+    const uint32_t cd1 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
+    c[0] = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u);
+    c[1] = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
+    c[2] = __builtin_amdgcn_perm(cd1, ab1, 0x05040100u);
+    c[3] = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
+}
+
+// 0x80 in every byte of x that is >= limit (1 <= limit <= 255)
+__device__ __forceinline__ uint32_t bytes_at_least(uint32_t x, uint32_t limit) {
+    const uint32_t low = x & 0x7f7f7f7fu;
+    const uint32_t hit = limit <= 128u ? ((low + (128u - limit) * 0x01010101u) | x)
+                                       : ((low + (256u - limit) * 0x01010101u) & x);
+    return hit & 0x80808080u;
+}
+
+__global__ __launch_bounds__(kBlock) void transpose_bins_kernel(const uint8_t* __restrict__ src, int64_t n,
+                                                            int64_t stride, int32_t F,
+                                                            const int64_t* __restrict__ perm,
+                                                            uint8_t* __restrict__ out, int64_t n_out, int64_t ld,
+                                                            int32_t ftiles, uint32_t limit,
+                                                            int32_t* __restrict__ over) {
+    __shared__ uint32_t tile[kTrFeats][kTrRows / 4 + 1];
+    const int64_t r0 = (int64_t)(blockIdx.x / (uint32_t)ftiles) * kTrRows;
+    const int f0 = (int)(blockIdx.x % (uint32_t)ftiles) * kTrFeats;
+    const int fg = threadIdx.x & 7;  // 16-feature group
+    const int f = f0 + fg * 16;
+    constexpr int kIt = kTrRows / 128;  // row quads per thread: rows r0 + 4 rq .. for rq = tid / 8 + 32 it
+    Bytes16 v[kIt][4];
+    if (r0 + kTrRows <= n && f0 + kTrFeats <= F) {  // uniform: no guard, every load in flight at once
+        const int64_t rb = r0 + 4 * (int)(threadIdx.x >> 3);
+#pragma unroll
+        for (int it = 0; it < kIt; ++it)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t r = rb + 128 * it + i;
+                v[it][i] = *reinterpret_cast<const Bytes16*>(src + (perm ? perm[r] : r) * stride + f);
+            }
+    } else {
+#pragma unroll
+        for (int it = 0; it < kIt; ++it)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t r = r0 + 4 * ((int)(threadIdx.x >> 3) + 32 * it) + i;
+                v[it][i] = Bytes16{{0u, 0u, 0u, 0u}};
+                if (r >= n || f >= F) continue;
+                const uint8_t* p = src + (perm ? perm[r] : r) * stride + f;
+                if (f + 16 <= F) {
+                    v[it][i] = *reinterpret_cast<const Bytes16*>(p);
+                } else {  // the last features of a row: no byte past the row is read
+#pragma unroll
+                    for (int b = 0; b < 16; ++b)
+                        if (b < F - f) v[it][i].w[b >> 2] |= (uint32_t)p[b] << (8 * (b & 3));
+                }
+            }
+    }
+    uint32_t hit = 0u;
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+        const int rq = (int)(threadIdx.x >> 3) + it * 32;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t rows4[4] = {v[it][0].w[q], v[it][1].w[q], v[it][2].w[q], v[it][3].w[q]};
+            uint32_t cols4[4];
+            transpose4x4_bytes(rows4, cols4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (limit) hit |= bytes_at_least(cols4[k], limit);
+                tile[fg * 16 + q * 4 + k][rq] = cols4[k];
+            }
+        }
+    }
+    if (limit && hit) atomicOr(over, 1);
+    __syncthreads();
+    // 16 lanes per column, 16 bytes (16 rows) each
+    const int q = threadIdx.x & 15;
+    const int64_t row = r0 + 16 * q;
+    if (row >= n_out) return;
+#pragma unroll
+    for (int it = 0; it < kTrFeats / 16; ++it) {
+        const int k = (int)(threadIdx.x >> 4) + it * 16;
+        if (f0 + k >= F) break;
+        const uint4 w = make_uint4(tile[k][4 * q], tile[k][4 * q + 1], tile[k][4 * q + 2], tile[k][4 * q + 3]);
+        *reinterpret_cast<uint4*>(out + (int64_t)(f0 + k) * ld + row) = w;
+    }
+}
+
 }  // namespace
+
+hipError_t launch_transpose_bins(const uint8_t* src, int64_t n, int64_t stride, int32_t F, const int64_t* perm,
+                                 uint8_t* out, int64_t n_out, int64_t ld, int32_t limit, int32_t* over,
+                                 hipStream_t s) {
+    const int64_t ftiles = (F + kTrFeats - 1) / kTrFeats;
+    const int64_t grid = (n_out + kTrRows - 1) / kTrRows * ftiles;
+    if (grid > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(transpose_bins_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, src, n, stride, F, perm,
+                       out, n_out, ld, (int32_t)ftiles, (uint32_t)limit, over);
+    return hipGetLastError();
+}
 
 hipError_t launch_pack_bins4(const uint8_t* bins, int64_t n, int64_t ld, int32_t F, uint8_t* out,
                              hipStream_t s) {

@@ -1048,6 +1048,23 @@ int pb_apply_bins(const float* xt, int64_t n, int64_t ld_x, int32_t F, const flo
     return PB_OK;
 }
 
+int pb_transpose_bins(const uint8_t* src, int64_t n, int64_t row_stride, int32_t F, const int64_t* perm,
+                      uint8_t* out, int64_t n_out, int64_t ld, int32_t limit, int32_t* over, void* stream) {
+    if (n < 0 || F < 0 || row_stride < 0 || n_out < n || ld < n_out || n_out % 16 != 0 || ld % 16 != 0)
+        return fail(PB_ERR_INVALID, "pb_transpose_bins: n <= n_out <= ld, n_out and ld multiples of 16");
+    if (limit < 0 || limit > 255) return fail(PB_ERR_INVALID, "pb_transpose_bins: limit must lie in [0, 255]");
+    if (n_out == 0 || F == 0) return PB_OK;
+    if ((!src && n > 0) || !out || (limit > 0 && !over))
+        return fail(PB_ERR_INVALID, "pb_transpose_bins: null argument");
+    if (reinterpret_cast<uintptr_t>(out) & 15)
+        return fail(PB_ERR_INVALID, "pb_transpose_bins: out must be 16-byte aligned");
+    if ((n_out + 255) / 256 * ((F + 127) / 128) > INT32_MAX)
+        return fail(PB_ERR_UNSUPPORTED, "pb_transpose_bins: grid too large");
+    PB_HIP(pb::launch_transpose_bins(src, n, row_stride, F, perm, out, n_out, ld, limit, over, (hipStream_t)stream),
+           "transpose bins launch");
+    return PB_OK;
+}
+
 int pb_pack_bins4(const uint8_t* bins, int64_t n, int64_t ld, int32_t F, uint8_t* out, void* stream) {
     if (!bins || !out) return fail(PB_ERR_INVALID, "pb_pack_bins4: null argument");
     if (ld < 0 || ld % 16 != 0 || F < 0) return fail(PB_ERR_INVALID, "pb_pack_bins4: ld must be a multiple of 16");

@@ -370,6 +370,9 @@ hipError_t launch_round_begin(const float* preds, const float* y, float* grad, u
 hipError_t launch_round_end(const uint16_t* tnode, const float* values, int32_t pack_size,
                             float lr, float* preds, int64_t N, const Frontier* st, pb_round_header* header,
                             hipStream_t s);
+hipError_t launch_transpose_bins(const uint8_t* src, int64_t n, int64_t stride, int32_t F, const int64_t* perm,
+                                 uint8_t* out, int64_t n_out, int64_t ld, int32_t limit, int32_t* over,
+                                 hipStream_t s);
 hipError_t launch_pack_bins4(const uint8_t* bins, int64_t n, int64_t ld, int32_t F, uint8_t* out,
                              hipStream_t s);
 // Row-list kernels (rowlist.hip). Workspace: rowlist_work_elems(segments) int32, whose first
