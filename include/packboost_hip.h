@@ -389,6 +389,13 @@ int pb_forest_create(const int32_t* feature_dev, const int32_t* threshold_dev,
 int pb_forest_predict(const pb_forest* forest, const uint8_t* bins_dev, int64_t N, int64_t ld,
                       int32_t F, float tree_weight, float* out_dev, int32_t* leaf_dev,
                       void* stream);
+/* pb_forest_predict on row-major bins (row r's features adjacent at rows_dev + r * row_stride, any
+ * alignment), by the tiled walk: the same sums and leaf indices, without a column-major copy.
+ * pb_forest_takes_rows: 1 if the forest has a tiled walk, else 0 (and pb_forest_predict_rows
+ * returns PB_ERR_UNSUPPORTED). */
+int32_t pb_forest_takes_rows(const pb_forest* forest);
+int pb_forest_predict_rows(const pb_forest* forest, const uint8_t* rows_dev, int64_t N, int64_t row_stride,
+                           int32_t F, float tree_weight, float* out_dev, int32_t* leaf_dev, void* stream);
 int pb_forest_destroy(pb_forest* forest);
 
 /* Single tree. Replaces predict_bins_cuda (frontier_cuda.cu:193-233, 853-920):

@@ -36,7 +36,8 @@ EXPORTED_SYMBOLS = (
     "pb_forest_create", "pb_forest_predict", "pb_forest_destroy", "pb_pack_bins4",
     "pb_set_bin_layout", "pb_select_subsets", "pb_rowlist_work_elems", "pb_rowlist_partition",
     "pb_rowlist_gather", "pb_best_thresholds", "pb_pick_sequential", "pb_set_segment_mode", "pb_rowlist_noalloc_max_segments",
-    "pb_rowlist_partition_noalloc", "pb_transpose_bins",
+    "pb_rowlist_partition_noalloc", "pb_transpose_bins", "pb_forest_takes_rows",
+    "pb_forest_predict_rows",
 )
 
 
@@ -114,6 +115,8 @@ _SIGNATURES = {
     "pb_era_corr": (ctypes.c_int, [_VP, _VP, _VP, _I32, _VP, _VP, _VP]),
     "pb_forest_create": (ctypes.c_int, [_VP] * 7 + [_I32, _I32, _VP]),
     "pb_forest_predict": (ctypes.c_int, [_VP, _VP, _I64, _I64, _I32, _F32, _VP, _VP, _VP]),
+    "pb_forest_takes_rows": (_I32, [_VP]),
+    "pb_forest_predict_rows": (ctypes.c_int, [_VP, _VP, _I64, _I64, _I32, _F32, _VP, _VP, _VP]),
     "pb_forest_destroy": (ctypes.c_int, [_VP]),
     "pb_quantile_edges": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _VP, _I32, _VP]),
     "pb_apply_bins": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _I32, _I32, _VP, _VP, _I64, _VP]),

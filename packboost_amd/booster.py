@@ -120,17 +120,19 @@ def _device_of(x) -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
-def _to_column_major(bins, device: torch.device) -> torch.Tensor:
-    """Row-major integer bins [N, F] (numpy or torch) -> contiguous uint8 [F, ld] on device."""
-    if isinstance(bins, torch.Tensor):
-        t = bins
-    else:
-        t = torch.from_numpy(np.ascontiguousarray(bins))
+def _u8_rows(bins, device: torch.device) -> torch.Tensor:
+    """Row-major integer bins [N, F] (numpy or torch) as uint8 on the device."""
+    t = bins if isinstance(bins, torch.Tensor) else torch.from_numpy(np.ascontiguousarray(bins))
     if t.dtype not in (torch.uint8, torch.int8):
         t = t.to(torch.uint8)
+    return t.to(device).view(torch.uint8)
+
+
+def _to_column_major(bins, device: torch.device) -> torch.Tensor:
+    """Row-major integer bins [N, F] (numpy or torch) -> contiguous uint8 [F, ld] on device."""
+    t = _u8_rows(bins, device)
     N, F = t.shape
     out = torch.empty((int(F), padded_rows(int(N))), dtype=torch.uint8, device=device)
-    t = t.to(device).view(torch.uint8)
     if not transpose_rows(t, out):
         out[:, :N] = t.t()
         out[:, N:] = 0
@@ -152,15 +154,34 @@ def _bins_fm_for(X, bin_edges, max_bins: int, device: torch.device,
     if bin_edges is not None and _is_float_input(X):
         out = apply_bins_device(X, bin_edges, max_bins, device, perm=perm)
         return out, int(X.shape[0])
-    if isinstance(X, torch.Tensor):
-        if X.dtype.is_floating_point:
-            raise ValueError("float inputs need the model's bin edges (the model was trained on bins)")
-        bins = X if perm is None else X[torch.as_tensor(perm, device=X.device)]
-    else:
-        bins = apply_bins(X, bin_edges, max_bins)
-        if perm is not None:
-            bins = bins[perm]
+    bins = _integer_bins(X, bin_edges, max_bins)
+    if perm is not None:
+        bins = bins[torch.as_tensor(perm, device=bins.device) if isinstance(bins, torch.Tensor) else perm]
     return _to_column_major(bins, device), int(bins.shape[0])
+
+
+def _integer_bins(X, bin_edges, max_bins: int):
+    """The bins of an integer input: a tensor is taken as bins, an array by apply_bins' rule."""
+    if not isinstance(X, torch.Tensor):
+        return apply_bins(X, bin_edges, max_bins)
+    if X.dtype.is_floating_point:
+        raise ValueError("float inputs need the model's bin edges (the model was trained on bins)")
+    return X
+
+
+def _forest_predict(forest, X, bin_edges, max_bins: int, device: torch.device, tree_weight: float,
+                    leaves: torch.Tensor | None = None) -> torch.Tensor:
+    """A compiled forest's predictions (and leaves) for rows X as _bins_fm_for takes them. Integer
+    bins whose features are adjacent go to the tiled walk as they lie (it stages each row once: a
+    column-major copy would move every bin three times); floats, other layouts and forests
+    without a tiled walk go through column-major bins."""
+    if not (bin_edges is not None and _is_float_input(X)):
+        rows = _u8_rows(_integer_bins(X, bin_edges, max_bins), device)
+        if forest.takes_rows() and (rows.shape[1] == 1 or rows.stride(1) == 1):
+            return forest.predict_rows(rows, tree_weight, leaves)
+        return forest.predict(_to_column_major(rows, device), int(rows.shape[0]), tree_weight, leaves)
+    bins_fm, n = _bins_fm_for(X, bin_edges, max_bins, device)
+    return forest.predict(bins_fm, n, tree_weight, leaves)
 
 
 def _require_backend(device: torch.device) -> None:
@@ -398,8 +419,8 @@ class PackBoost:
             raise RuntimeError("Missing _tree_weight; call fit() first.")
         device = self._device if self._device.index is not None else torch.device(
             "cuda", torch.cuda.current_device())
-        bins_fm, N = _bins_fm_for(X, self._binner.bin_edges, self.config.max_bins, device)
-        out = self._predict_device(bins_fm, N, device)
+        out = _forest_predict(self._compiled(device), X, self._binner.bin_edges, self.config.max_bins, device,
+                              float(self._tree_weight))
         return out.cpu().numpy()
 
     def save(self, path) -> "Path":
@@ -425,7 +446,7 @@ class PackBoost:
         self._forest_cache = (key, forest)
         return forest
 
-    def _predict_device(self, bins_fm: torch.Tensor, N: int, device: torch.device) -> torch.Tensor:
+    def _compiled(self, device: torch.device):
         from .predictor import CompiledForest
 
         key = (str(device), len(self._rounds))
@@ -433,7 +454,10 @@ class PackBoost:
         if cached is None or cached[0] != key:
             cached = (key, CompiledForest(self._forest_device(device)))
             self._compiled_forest = cached
-        return cached[1].predict(bins_fm, N, float(self._tree_weight))
+        return cached[1]
+
+    def _predict_device(self, bins_fm: torch.Tensor, N: int, device: torch.device) -> torch.Tensor:
+        return self._compiled(device).predict(bins_fm, N, float(self._tree_weight))
 
     def _prepare_eval(self, eval_sets, device) -> list[dict]:
         states = []

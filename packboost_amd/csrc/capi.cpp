@@ -1331,7 +1331,7 @@ int pb_forest_predict(const pb_forest* fo, const uint8_t* bins, int64_t N, int64
     // the tiled walk reads a tile's rows four at a time: row stride and columns 4-byte aligned
     if (fo->heap_blocks && ld % 4 == 0 && reinterpret_cast<uintptr_t>(bins) % 4 == 0 &&
         env_int("PB_FOREST_TILE", 1) != 0) {
-        PB_HIP(pb::launch_forest_tile(bins, N, ld, fo->tile, fo->heap_blocks, fo->heap_id, fo->heap_first,
+        PB_HIP(pb::launch_forest_tile(bins, N, ld, 0, fo->tile, fo->heap_blocks, fo->heap_id, fo->heap_first,
                                       fo->heap_trees, fo->depth, tree_weight, out, leaf, (hipStream_t)stream),
                "forest tile launch");
         return PB_OK;
@@ -1341,6 +1341,26 @@ int pb_forest_predict(const pb_forest* fo, const uint8_t* bins, int64_t N, int64
     PB_HIP(pb::launch_forest(bins, N, ld, fo->rec, fo->roots, fo->T, fo->depth, tree_weight, out, leaf,
                              group, max_grid, (hipStream_t)stream),
            "forest launch");
+    return PB_OK;
+}
+
+int32_t pb_forest_takes_rows(const pb_forest* fo) {
+    return fo && fo->heap_blocks && env_int("PB_FOREST_TILE", 1) != 0 ? 1 : 0;
+}
+
+int pb_forest_predict_rows(const pb_forest* fo, const uint8_t* rows, int64_t N, int64_t row_stride, int32_t F,
+                           float tree_weight, float* out, int32_t* leaf, void* stream) {
+    if (!fo) return fail(PB_ERR_INVALID, "pb_forest_predict_rows: null forest");
+    if (N < 0 || F < 1 || row_stride < 0) return fail(PB_ERR_INVALID, "pb_forest_predict_rows: bad shape");
+    if (fo->max_feature >= F)
+        return fail(PB_ERR_RANGE, "pb_forest_predict_rows: the forest splits on a feature >= F");
+    if (!pb_forest_takes_rows(fo))
+        return fail(PB_ERR_UNSUPPORTED, "pb_forest_predict_rows: the forest has no tiled walk");
+    if (N == 0) return PB_OK;
+    if (!rows || !out) return fail(PB_ERR_INVALID, "pb_forest_predict_rows: null argument");
+    PB_HIP(pb::launch_forest_tile(rows, N, row_stride, F, fo->tile, fo->heap_blocks, fo->heap_id, fo->heap_first,
+                                  fo->heap_trees, fo->depth, tree_weight, out, leaf, (hipStream_t)stream),
+           "forest tile launch");
     return PB_OK;
 }
 

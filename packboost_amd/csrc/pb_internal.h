@@ -438,7 +438,9 @@ struct ForestTile {
 ForestTile forest_tile_shape(int32_t features, int32_t max_threshold, int32_t depth, int32_t trees);
 size_t forest_tile_lds_bytes(const ForestTile& ft);
 uint32_t forest_tile_record(const ForestTile& ft, int32_t feature, int32_t threshold);
-hipError_t launch_forest_tile(const uint8_t* bins, int64_t N, int64_t ld, const ForestTile& ft,
+// row_feats 0: column-major bins of row stride ld; else row-major bins of row_feats features, ld bytes
+// from row to row.
+hipError_t launch_forest_tile(const uint8_t* bins, int64_t N, int64_t ld, int32_t row_feats, const ForestTile& ft,
                               const uint32_t* blocks, const int32_t* lid, const int32_t* tfirst, int32_t T,
                               int32_t depth, float tree_weight, float* out, int32_t* leaf, hipStream_t s);
 hipError_t launch_predict_pack(const uint8_t* bins, int64_t N, int64_t ld, int32_t F,

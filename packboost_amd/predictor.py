@@ -128,6 +128,21 @@ class CompiledForest:
             "pb_forest_predict")
         return out
 
+    def takes_rows(self) -> bool:
+        """Whether predict_rows serves this forest (it has a tiled walk)."""
+        return bool(self._lib.pb_forest_takes_rows(self._h))
+
+    def predict_rows(self, rows: torch.Tensor, tree_weight: float,
+                     leaves: torch.Tensor | None = None) -> torch.Tensor:
+        """predict() of row-major uint8 bins [N, F] on the device, features adjacent."""
+        n = int(rows.shape[0])
+        out = torch.empty(n, dtype=torch.float32, device=rows.device)
+        _hip.check(self._lib.pb_forest_predict_rows(
+            self._h, rows.data_ptr(), n, rows.stride(0), int(rows.shape[1]), float(tree_weight),
+            out.data_ptr(), None if leaves is None else leaves.data_ptr(), _hip.stream_ptr()),
+            "pb_forest_predict_rows")
+        return out
+
     def close(self) -> None:
         if getattr(self, "_h", None) is not None and self._h.value:
             torch.cuda.synchronize()
@@ -187,29 +202,31 @@ class PackBoostPredictor:
             self._cforest = CompiledForest(self._packed())
         return self._cforest
 
-    def _bins_fm(self, X) -> tuple[torch.Tensor, int]:
-        from .booster import _bins_fm_for
+    def _walk(self, X, leaves: bool = False) -> tuple[torch.Tensor, torch.Tensor | None] | None:
+        """Predictions (and absolute leaf indices) on the device, or None where there is no row or
+        no tree (the input is checked all the same)."""
+        from .booster import _bins_fm_for, _forest_predict
 
-        nf = int(X.shape[1])
+        n, nf = int(X.shape[0]), int(X.shape[1])
         if self.feature_names and nf != len(self.feature_names):
             raise ValueError(f"X has {nf} features; the model expects {len(self.feature_names)}")
-        return _bins_fm_for(X, self.bin_edges, self.config.max_bins, self.device)
+        if n == 0 or self.num_trees == 0:
+            _bins_fm_for(X, self.bin_edges, self.config.max_bins, self.device)
+            return None
+        cf = self._compiled()
+        leaf = torch.empty((self.num_trees, n), dtype=torch.int32, device=self.device) if leaves else None
+        return _forest_predict(cf, X, self.bin_edges, self.config.max_bins, self.device, self.tree_weight, leaf), leaf
 
     def predict(self, X) -> np.ndarray:
         """float32 predictions, bit-identical to PackBoost.predict on the same model."""
-        bins_fm, n = self._bins_fm(X)
-        if not self.rounds or n == 0:
-            return np.zeros(n, dtype=np.float32)
-        return self._compiled().predict(bins_fm, n, self.tree_weight).cpu().numpy()
+        got = self._walk(X)
+        return np.zeros(int(X.shape[0]), dtype=np.float32) if got is None else got[0].cpu().numpy()
 
     def predict_leaves(self, X) -> np.ndarray:
         """int32 [num_trees, N]: each tree's leaf, as a node index within that tree."""
-        bins_fm, n = self._bins_fm(X)
-        T = self.num_trees
-        if T == 0 or n == 0:
-            return np.zeros((T, n), dtype=np.int32)
-        cf = self._compiled()
-        leaf = torch.empty((T, n), dtype=torch.int32, device=self.device)
-        cf.predict(bins_fm, n, self.tree_weight, leaves=leaf)
+        got = self._walk(X, leaves=True)
+        if got is None:
+            return np.zeros((self.num_trees, int(X.shape[0])), dtype=np.int32)
+        cf, leaf = self._compiled(), got[1]
         offs = cf.offsets[:-1].to(torch.int32)[:, None]
         return (leaf - offs).cpu().numpy()

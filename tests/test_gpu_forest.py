@@ -139,3 +139,35 @@ def test_forest_rejects_malformed(hip):
                               1, int(f["value"].numel()), ctypes.byref(h))
     assert rc == -1 and not h.value
     assert b"malformed" in lib.pb_last_error()
+
+
+@pytest.mark.parametrize("D,F,max_thr,N", [
+    (0, 1, 3, 5), (3, 9, 3, 63), (6, 239, 6, 64), (5, 240, 6, 65), (6, 241, 5, 1000), (4, 480, 14, 129),
+    (3, 481, 14, 64), (2, 15, 200, 31), (5, 700, 200, 333), (7, 2376, 255, 97), (6, 2376, 3, 2049)])
+def test_rows_walk(hip, D, F, max_thr, N):
+    """The tiled walk staged from row-major bins (every packing, 32- and 64-row tiles, chunk and
+    row-tile edges, unaligned rows and strides, bins above the packed fields) against the walk of
+    column-major bins: the same sums in the same order, so equal bit for bit, leaves included."""
+    import torch
+
+    from packboost_amd.booster import _to_column_major, pack_forest
+    from packboost_amd.predictor import CompiledForest
+
+    rounds = _forest(21 + D, 7, 3, D, F, ragged=True, max_thr=max_thr)
+    g = torch.Generator(device="cuda").manual_seed(D + F)
+    wide = torch.randint(0, 256, (N, F + 7), dtype=torch.uint8, device="cuda", generator=g)
+    low = torch.randint(0, max_thr + 2, (N, F + 7), device="cuda", generator=g).clamp(max=255).to(torch.uint8)
+    cf = CompiledForest(pack_forest(rounds, 3, torch.device("cuda")))
+    assert cf.takes_rows()
+    for base in (wide, low):
+        for rows in (base[:, 5:5 + F], base[:, :F].contiguous()):
+            want_l, got_l = (torch.empty((21, N), dtype=torch.int32, device="cuda") for _ in range(2))
+            want = cf.predict(_to_column_major(rows, torch.device("cuda")), N, 0.5, leaves=want_l)
+            got = cf.predict_rows(rows, 0.5, leaves=got_l)
+            assert torch.equal(got, want) and torch.equal(got_l, want_l)
+            assert torch.equal(cf.predict_rows(rows, 0.5), want)
+    top = max(int(r["feature"].max()) for r in rounds)
+    if top > 0:
+        with pytest.raises(hip.HipBackendError, match="feature >= F"):
+            cf.predict_rows(wide[:, :top], 0.5)
+    cf.close()
