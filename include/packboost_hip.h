@@ -324,6 +324,15 @@ int pb_transpose_bins(const uint8_t* src_dev, int64_t n, int64_t row_stride, int
                       uint8_t* out_dev, int64_t n_out, int64_t ld, int32_t limit, int32_t* over_dev,
                       void* stream);
 
+/* apply_bins (data.py:93-111) of row-major values to the frontier kernels' bins: out_dev[f][r] =
+ * min(searchsorted(edges[:, f], x, side="left"), max_bins - 1) with NumPy's NaN-last order and
+ * edges ascending in it, x = x_dev[(perm_dev ? perm_dev[r] : r) * row_stride + f] (strides in
+ * elements), for r < n; 0 for rows n .. n_out-1. edges_dev: float32 [num_edges][edge_stride],
+ * num_edges <= 254. n <= n_out <= ld, n_out % 16 == ld % 16 == 0; out_dev 16-byte aligned. */
+int pb_bin_rows(const float* x_dev, int64_t n, int64_t row_stride, int32_t F, const float* edges_dev,
+                int32_t num_edges, int32_t edge_stride, int32_t max_bins, const int64_t* perm_dev, uint8_t* out_dev,
+                int64_t n_out, int64_t ld, void* stream);
+
 /* apply_bins (data.py:93-111): bins[f][r] = min(searchsorted(edges[:, f], x, side="left"),
  * max_bins - 1) with NumPy's NaN-last order, x = xt[f][perm ? perm[r] : r] (xt: float32
  * [F][ld_x] column-major values; perm: optional int64 [n] row gather, e.g. the era-major

@@ -1048,6 +1048,21 @@ int pb_apply_bins(const float* xt, int64_t n, int64_t ld_x, int32_t F, const flo
     return PB_OK;
 }
 
+int pb_bin_rows(const float* x, int64_t n, int64_t row_stride, int32_t F, const float* edges, int32_t num_edges,
+                int32_t edge_stride, int32_t max_bins, const int64_t* perm, uint8_t* out, int64_t n_out, int64_t ld,
+                void* stream) {
+    if (n < 0 || F < 0 || row_stride < 0 || n_out < n || ld < n_out || n_out % 16 != 0 || ld % 16 != 0 ||
+        num_edges < 1 || num_edges > 254 || edge_stride < F || max_bins < 2 || max_bins > 255)
+        return fail(PB_ERR_INVALID, "pb_bin_rows: bad shape");
+    if (n_out == 0 || F == 0) return PB_OK;
+    if ((!x && n > 0) || !edges || !out) return fail(PB_ERR_INVALID, "pb_bin_rows: null argument");
+    if (reinterpret_cast<uintptr_t>(out) & 15) return fail(PB_ERR_INVALID, "pb_bin_rows: out must be 16-byte aligned");
+    PB_HIP(pb::launch_bin_rows(x, n, row_stride, F, edges, num_edges, edge_stride, max_bins, perm, out, n_out, ld,
+                               (hipStream_t)stream),
+           "bin rows launch");
+    return PB_OK;
+}
+
 int pb_transpose_bins(const uint8_t* src, int64_t n, int64_t row_stride, int32_t F, const int64_t* perm,
                       uint8_t* out, int64_t n_out, int64_t ld, int32_t limit, int32_t* over, void* stream) {
     if (n < 0 || F < 0 || row_stride < 0 || n_out < n || ld < n_out || n_out % 16 != 0 || ld % 16 != 0)

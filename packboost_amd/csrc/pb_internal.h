@@ -370,6 +370,9 @@ hipError_t launch_round_begin(const float* preds, const float* y, float* grad, u
 hipError_t launch_round_end(const uint16_t* tnode, const float* values, int32_t pack_size,
                             float lr, float* preds, int64_t N, const Frontier* st, pb_round_header* header,
                             hipStream_t s);
+hipError_t launch_bin_rows(const float* x, int64_t n, int64_t stride, int32_t F, const float* edges, int32_t ne,
+                           int32_t edge_stride, int32_t max_bins, const int64_t* perm, uint8_t* out,
+                           int64_t n_out, int64_t ld, hipStream_t s);
 hipError_t launch_transpose_bins(const uint8_t* src, int64_t n, int64_t stride, int32_t F, const int64_t* perm,
                                  uint8_t* out, int64_t n_out, int64_t ld, int32_t limit, int32_t* over,
                                  hipStream_t s);

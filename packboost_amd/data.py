@@ -10,7 +10,7 @@ Semantics follow the reference's packboost/data.py:
 Bins are returned as uint8 (values identical to the reference's int8 for max_bins <= 128).
 
 quantile_bin_device / apply_bins_device do the same on the HIP device (pb_quantile_edges,
-pb_apply_bins) and write the histogram kernel's column-major layout directly; their edges and
+pb_bin_rows) and write the histogram kernel's column-major layout directly; their edges and
 bins are bit-identical to the NumPy path.
 """
 
@@ -149,11 +149,15 @@ def feature_names_or_default(feature_names: Sequence[str] | None, n_features: in
 
 
 def _float_matrix_device(X, device):
+    """float32 [N, F] on the device: a row's features adjacent, or a feature's rows."""
     import torch
 
     if isinstance(X, torch.Tensor):
-        return X.detach().to(device=device, dtype=torch.float32).contiguous()
-    Xn = np.ascontiguousarray(ensure_numpy(X), dtype=np.float32)
+        x = X.detach().to(device=device, dtype=torch.float32)
+        return x if x.dim() == 2 and 1 in x.stride() else x.contiguous()
+    Xn = np.asarray(ensure_numpy(X), dtype=np.float32)
+    if not (Xn.flags.c_contiguous or Xn.flags.f_contiguous):
+        Xn = np.ascontiguousarray(Xn)
     return torch.from_numpy(Xn).to(device)
 
 
@@ -169,33 +173,36 @@ def _device_bins(X, max_bins: int, device, perm, edges, chunk_features: int):
     N, F = int(x.shape[0]), int(x.shape[1])
     ld = (N + 15) // 16 * 16
     nq = int(max_bins) - 1
-    out = torch.zeros((F, ld), dtype=torch.uint8, device=device)
+    out = torch.empty((F, ld), dtype=torch.uint8, device=device)
     perm_dev = None
     if perm is not None:
         perm_dev = torch.as_tensor(np.ascontiguousarray(perm, dtype=np.int64)).to(device)
+    s = _hip.stream_ptr()
     if edges is None:
         qs = np.linspace(0.0, 1.0, int(max_bins) + 1, dtype=np.float64)[1:-1]
         q_dev = torch.from_numpy(np.ascontiguousarray(qs)).to(device)
         edges_dev = torch.empty((nq, F), dtype=torch.float32, device=device)
+        for f0 in range(0, F, chunk_features):
+            f1 = min(F, f0 + chunk_features)
+            xt = x[:, f0:f1].t().contiguous()  # [fc, N] column values, a view of feature-major X
+            srt = torch.sort(xt, dim=1).values  # ascending, NaN last
+            _hip.check(lib.pb_quantile_edges(srt.data_ptr(), N, N, f1 - f0, q_dev.data_ptr(), nq,
+                                             edges_dev.data_ptr() + 4 * f0, F, s), "pb_quantile_edges")
+            del xt, srt
     else:
-        q_dev = None
         edges_dev = torch.from_numpy(np.ascontiguousarray(edges, dtype=np.float32)).to(device)
         if tuple(edges_dev.shape) != (nq, F):
             raise ValueError(f"bin_edges must be [{nq}, {F}]")
-    s = _hip.stream_ptr()
-    for f0 in range(0, F, chunk_features):
-        f1 = min(F, f0 + chunk_features)
-        xt = x[:, f0:f1].t().contiguous()  # [fc, N] column values
-        e_ptr = edges_dev.data_ptr() + 4 * f0
-        if q_dev is not None:
-            srt = torch.sort(xt, dim=1).values  # ascending, NaN last
-            _hip.check(lib.pb_quantile_edges(srt.data_ptr(), N, N, f1 - f0, q_dev.data_ptr(), nq,
-                                             e_ptr, F, s), "pb_quantile_edges")
-            del srt
-        _hip.check(lib.pb_apply_bins(xt.data_ptr(), N, N, f1 - f0, e_ptr, nq, F, int(max_bins),
-                                     None if perm_dev is None else perm_dev.data_ptr(),
-                                     out[f0].data_ptr(), ld, s), "pb_apply_bins")
-        del xt
+    if F == 1 or x.stride(1) == 1:
+        _hip.check(lib.pb_bin_rows(x.data_ptr(), N, x.stride(0), F, edges_dev.data_ptr(), nq, F, int(max_bins),
+                                   _hip.ptr(perm_dev), out.data_ptr(), ld, ld, s), "pb_bin_rows")
+    else:  # feature-major values: each column as it lies
+        out[:, N:] = 0
+        for f0 in range(0, F, chunk_features):
+            f1 = min(F, f0 + chunk_features)
+            _hip.check(lib.pb_apply_bins(x[:, f0:].data_ptr(), N, x.stride(1), f1 - f0,
+                                         edges_dev.data_ptr() + 4 * f0, nq, F, int(max_bins), _hip.ptr(perm_dev),
+                                         out[f0].data_ptr(), ld, s), "pb_apply_bins")
     return out, (edges_dev.cpu().numpy() if edges is None else np.asarray(edges, np.float32))
 
 

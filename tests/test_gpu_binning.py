@@ -93,3 +93,35 @@ def test_device_binning_matches_reference_golden(hip):
         np.testing.assert_array_equal(db, d["bins"], err_msg=name)
         want = d["edges"].reshape(len(d["edge_lens"]), -1).astype(np.float32)  # [max_bins - 1, F]
         assert_edges_equal(de, want, name)
+
+
+@pytest.mark.parametrize("n,f,nb", [(1, 1, 2), (127, 31, 3), (128, 32, 4), (129, 33, 17), (1000, 70, 129),
+                                    (5001, 5, 255), (300_000, 40, 64)])
+def test_bin_rows_shapes(hip, n, f, nb):
+    """Tile, feature-group and search-depth edges, strided and feature-major inputs, with and
+    without a row gather: bins equal NumPy's searchsorted (values on the edges, signed zeros,
+    infinities and NaN included), padding rows 0."""
+    import torch
+
+    from packboost_amd.data import apply_bins_device
+
+    rng = np.random.default_rng(n + f)
+    edges = np.sort(np.round(rng.standard_normal((nb - 1, f)), 2).astype(np.float32), axis=0)
+    edges[edges == 0] = -0.0
+    X = np.round(rng.standard_normal((n, f)), 2).astype(np.float32) * 2
+    X[rng.random((n, f)) < 0.05] = np.nan
+    X[rng.random((n, f)) < 0.05] = np.inf
+    X[rng.random((n, f)) < 0.05] = -np.inf
+    X[rng.random((n, f)) < 0.05] = 0.0
+    want = np.empty((n, f), np.uint8)
+    for j in range(f):
+        want[:, j] = np.minimum(np.searchsorted(edges[:, j], X[:, j], side="left"), nb - 1)
+    perm = rng.permutation(n)
+    wide = torch.zeros((n, f + 3), device="cuda")
+    wide[:, 2:2 + f] = torch.from_numpy(X).cuda()
+    inputs = (X, np.asfortranarray(X), wide[:, 2:2 + f], torch.from_numpy(X).cuda().t().contiguous().t())
+    for x in inputs:
+        for p in (None, perm):
+            got = apply_bins_device(x, edges, nb, torch.device("cuda"), perm=p, chunk_features=9)
+            assert got.shape == (f, (n + 15) // 16 * 16) and not bool(got[:, n:].any())
+            np.testing.assert_array_equal(got[:, :n].cpu().numpy().T, want if p is None else want[p])
