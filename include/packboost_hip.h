@@ -324,6 +324,16 @@ int pb_transpose_bins(const uint8_t* src_dev, int64_t n, int64_t row_stride, int
                       uint8_t* out_dev, int64_t n_out, int64_t ld, int32_t limit, int32_t* over_dev,
                       void* stream);
 
+/* quantile_bin's edges (data.py:44-56) of F columns of values in any order: element (r, f) at
+ * x_dev[r * row_stride + f * col_stride], one of the two strides 1; q_dev, edges_dev and
+ * edge_stride as in pb_quantile_edges, whose edges these are (a zero edge is +0.0). work_dev:
+ * pb_quantile_work_bytes(n, F, num_q) bytes, 256-byte aligned (-1: n not in [1, 2^30], F not in
+ * [1, 65535] or num_q not in [1, 254]). */
+int64_t pb_quantile_work_bytes(int64_t n, int32_t F, int32_t num_q);
+int pb_column_quantiles(const float* x_dev, int64_t n, int64_t row_stride, int64_t col_stride, int32_t F,
+                        const double* q_dev, int32_t num_q, float* edges_dev, int32_t edge_stride, void* work_dev,
+                        int64_t work_bytes, void* stream);
+
 /* apply_bins (data.py:93-111) of row-major values to the frontier kernels' bins: out_dev[f][r] =
  * min(searchsorted(edges[:, f], x, side="left"), max_bins - 1) with NumPy's NaN-last order and
  * edges ascending in it, x = x_dev[(perm_dev ? perm_dev[r] : r) * row_stride + f] (strides in

@@ -37,7 +37,7 @@ EXPORTED_SYMBOLS = (
     "pb_set_bin_layout", "pb_select_subsets", "pb_rowlist_work_elems", "pb_rowlist_partition",
     "pb_rowlist_gather", "pb_best_thresholds", "pb_pick_sequential", "pb_set_segment_mode", "pb_rowlist_noalloc_max_segments",
     "pb_rowlist_partition_noalloc", "pb_transpose_bins", "pb_forest_takes_rows",
-    "pb_forest_predict_rows", "pb_bin_rows",
+    "pb_forest_predict_rows", "pb_bin_rows", "pb_quantile_work_bytes", "pb_column_quantiles",
 )
 
 
@@ -120,6 +120,8 @@ _SIGNATURES = {
     "pb_forest_destroy": (ctypes.c_int, [_VP]),
     "pb_quantile_edges": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _VP, _I32, _VP]),
     "pb_apply_bins": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _I32, _I32, _VP, _VP, _I64, _VP]),
+    "pb_quantile_work_bytes": (_I64, [_I64, _I32, _I32]),
+    "pb_column_quantiles": (ctypes.c_int, [_VP, _I64, _I64, _I64, _I32, _VP, _I32, _VP, _I32, _VP, _I64, _VP]),
     "pb_bin_rows": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _I32, _I32, _VP, _VP, _I64, _I64, _VP]),
     "pb_transpose_bins": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _VP, _I64, _I64, _I32, _VP, _VP]),
     "pb_pack_bins4": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _VP]),

@@ -21,6 +21,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_NAME = "libpackboost_hip.so"
 LIB_PATH = PKG_DIR / LIB_NAME
 SOURCES = ["hist.hip", "score.hip", "partition.hip", "predict.hip", "metrics.hip", "binning.hip", "rowlist.hip", "segment.hip",
+           "quantile.hip",
            "capi.cpp"]
 ARCH = "gfx950"
 

@@ -100,6 +100,8 @@ __device__ __forceinline__ uint32_t order_key(float x) {
 // feature) on distinct banks; the later ones are random. The LDS probes bound it
 // (a random one takes about 9 clocks): 1M x 500 values through 254 edges take 1.13 ms (440 G
 // values/s; 0.65 ms through 15 edges), where transposed copies and one search per lane took 9.0 ms.
+// Edges that do not ascend (a column with infinities between its quantiles has NaN edges below
+// finite ones) take searchsorted's own probe order instead, which decides what it finds there.
 // All feature groups of a row range run on one XCD, where its rows' split cache lines are shared.
 typedef __attribute__((address_space(3))) uint32_t lds_word;
 constexpr int kBrRows = 128;
@@ -115,6 +117,7 @@ __global__ __launch_bounds__(kBlock) void bin_rows_kernel(const float* __restric
     constexpr int kCap = (1 << STEPS) - 1, kStride = kCap + (STEPS == 1 ? 0 : 2);
     __shared__ uint32_t s_edge[kBrFeats * kStride];
     __shared__ uint32_t s_tile[kBrFeats][kBrRows / 4 + 1];
+    __shared__ uint32_t s_mixed;  // some feature's edges do not ascend
     const int64_t item = blockIdx.x >> 3;
     const int64_t chunk = item / groups * 8 + (blockIdx.x & 7);
     const int f0 = (int)(item % groups) * kBrFeats;
@@ -124,6 +127,12 @@ __global__ __launch_bounds__(kBlock) void bin_rows_kernel(const float* __restric
         const int fl = i & (kBrFeats - 1), e = i / kBrFeats;
         const bool in = e < ne && f0 + fl < F;
         s_edge[fl * kStride + e] = in ? order_key(edges[(int64_t)e * edge_stride + f0 + fl]) : 0xffffffffu;
+    }
+    if (threadIdx.x == 0) s_mixed = 0u;
+    __syncthreads();
+    for (int i = threadIdx.x; i < kBrFeats * (kCap - 1); i += kBlock) {
+        const int fl = i & (kBrFeats - 1), e = i / kBrFeats;
+        if (s_edge[fl * kStride + e] > s_edge[fl * kStride + e + 1]) s_mixed = 1u;
     }
     const int fq = threadIdx.x & 7, rq = threadIdx.x >> 3;
     const int f = f0 + 4 * fq;
@@ -162,6 +171,23 @@ __global__ __launch_bounds__(kBlock) void bin_rows_kernel(const float* __restric
                 key[i][k] = order_key(v[i].v[k]);
                 at[i][k] = edge0;
             }
+        if (s_mixed) {  // uniform
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t* edge = s_edge + (4 * fq + k) * kStride;
+                    int lo = 0, hi = ne;
+                    while (lo < hi) {
+                        const int mid = lo + ((hi - lo) >> 1);
+                        if (edge[mid] < key[i][k])
+                            lo = mid + 1;
+                        else
+                            hi = mid;
+                    }
+                    at[i][k] = edge0 + 4u * (uint32_t)lo;
+                }
+        } else
 #pragma unroll
         for (int s = STEPS - 1; s >= 0; --s)
 #pragma unroll

@@ -1048,6 +1048,27 @@ int pb_apply_bins(const float* xt, int64_t n, int64_t ld_x, int32_t F, const flo
     return PB_OK;
 }
 
+int64_t pb_quantile_work_bytes(int64_t n, int32_t F, int32_t num_q) {
+    if (n < 1 || n > pb::kMaxQuantileRows || F < 1 || F > 65535 || num_q < 1 || num_q > 254) return -1;
+    return pb::quantile_work_bytes(n, F, num_q);
+}
+
+int pb_column_quantiles(const float* x, int64_t n, int64_t row_stride, int64_t col_stride, int32_t F, const double* q,
+                        int32_t num_q, float* edges, int32_t edge_stride, void* work, int64_t work_bytes,
+                        void* stream) {
+    const int64_t need = pb_quantile_work_bytes(n, F, num_q);
+    if (need < 0 || row_stride < 0 || col_stride < 0 || (row_stride != 1 && col_stride != 1) || edge_stride < F)
+        return fail(PB_ERR_INVALID, "pb_column_quantiles: bad shape (1 <= n <= 2^30 rows, one stride 1)");
+    if (!x || !q || !edges || !work) return fail(PB_ERR_INVALID, "pb_column_quantiles: null argument");
+    if (work_bytes < need || (reinterpret_cast<uintptr_t>(work) & 255))
+        return fail(PB_ERR_INVALID, "pb_column_quantiles: the workspace must hold pb_quantile_work_bytes, "
+                                    "256-byte aligned");
+    PB_HIP(pb::launch_column_quantiles(x, n, row_stride, col_stride, F, q, num_q, edges, edge_stride, work,
+                                       (hipStream_t)stream),
+           "column quantiles launch");
+    return PB_OK;
+}
+
 int pb_bin_rows(const float* x, int64_t n, int64_t row_stride, int32_t F, const float* edges, int32_t num_edges,
                 int32_t edge_stride, int32_t max_bins, const int64_t* perm, uint8_t* out, int64_t n_out, int64_t ld,
                 void* stream) {

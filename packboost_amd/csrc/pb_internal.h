@@ -370,6 +370,13 @@ hipError_t launch_round_begin(const float* preds, const float* y, float* grad, u
 hipError_t launch_round_end(const uint16_t* tnode, const float* values, int32_t pack_size,
                             float lr, float* preds, int64_t N, const Frontier* st, pb_round_header* header,
                             hipStream_t s);
+// Quantile edges of F columns of x (element (r, f) at r * row_stride + f * col_stride, one of the
+// strides 1) by selection (quantile.hip), with quantile_work_bytes of workspace.
+constexpr int64_t kMaxQuantileRows = int64_t(1) << 30;
+int64_t quantile_work_bytes(int64_t n, int32_t F, int32_t nq);
+hipError_t launch_column_quantiles(const float* x, int64_t n, int64_t row_stride, int64_t col_stride, int32_t F,
+                                   const double* q, int32_t nq, float* edges, int32_t edge_stride, void* work,
+                                   hipStream_t s);
 hipError_t launch_bin_rows(const float* x, int64_t n, int64_t stride, int32_t F, const float* edges, int32_t ne,
                            int32_t edge_stride, int32_t max_bins, const int64_t* perm, uint8_t* out,
                            int64_t n_out, int64_t ld, hipStream_t s);

@@ -9,7 +9,7 @@ Semantics follow the reference's packboost/data.py:
   * build_era_index (data.py:114-134): per era, ascending row ids.
 Bins are returned as uint8 (values identical to the reference's int8 for max_bins <= 128).
 
-quantile_bin_device / apply_bins_device do the same on the HIP device (pb_quantile_edges,
+quantile_bin_device / apply_bins_device do the same on the HIP device (pb_column_quantiles,
 pb_bin_rows) and write the histogram kernel's column-major layout directly; their edges and
 bins are bit-identical to the NumPy path.
 """
@@ -184,11 +184,19 @@ def _device_bins(X, max_bins: int, device, perm, edges, chunk_features: int):
         edges_dev = torch.empty((nq, F), dtype=torch.float32, device=device)
         for f0 in range(0, F, chunk_features):
             f1 = min(F, f0 + chunk_features)
-            xt = x[:, f0:f1].t().contiguous()  # [fc, N] column values, a view of feature-major X
-            srt = torch.sort(xt, dim=1).values  # ascending, NaN last
-            _hip.check(lib.pb_quantile_edges(srt.data_ptr(), N, N, f1 - f0, q_dev.data_ptr(), nq,
-                                             edges_dev.data_ptr() + 4 * f0, F, s), "pb_quantile_edges")
-            del xt, srt
+            part = x[:, f0:f1]
+            e_ptr = edges_dev.data_ptr() + 4 * f0
+            size = int(lib.pb_quantile_work_bytes(N, f1 - f0, nq))
+            if size < 0:  # no rows, or more than the selection counts
+                srt = torch.sort(part.t().contiguous(), dim=1).values  # ascending, NaN last
+                _hip.check(lib.pb_quantile_edges(srt.data_ptr(), N, N, f1 - f0, q_dev.data_ptr(), nq, e_ptr, F, s),
+                           "pb_quantile_edges")
+                continue
+            work = torch.empty(size, dtype=torch.uint8, device=device)
+            by_row = F == 1 or x.stride(1) == 1
+            _hip.check(lib.pb_column_quantiles(part.data_ptr(), N, x.stride(0) if by_row else 1,
+                                               1 if by_row else x.stride(1), f1 - f0, q_dev.data_ptr(), nq, e_ptr, F,
+                                               work.data_ptr(), size, s), "pb_column_quantiles")
     else:
         edges_dev = torch.from_numpy(np.ascontiguousarray(edges, dtype=np.float32)).to(device)
         if tuple(edges_dev.shape) != (nq, F):

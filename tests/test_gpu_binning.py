@@ -125,3 +125,36 @@ def test_bin_rows_shapes(hip, n, f, nb):
             got = apply_bins_device(x, edges, nb, torch.device("cuda"), perm=p, chunk_features=9)
             assert got.shape == (f, (n + 15) // 16 * 16) and not bool(got[:, n:].any())
             np.testing.assert_array_equal(got[:, :n].cpu().numpy().T, want if p is None else want[p])
+
+
+@pytest.mark.parametrize("n,nb", [(1, 5), (2, 255), (3, 2), (16384, 128), (16385, 255), (16385, 2), (40_003, 63),
+                                  (530_001, 255)])
+def test_column_quantiles(hip, n, nb):
+    """The selection's edges equal NumPy's at its size limits (columns sorted in LDS up to 16384
+    rows, 255 splitters up to 2^19 rows, 1023 above) on columns that strain it: sorted and reversed
+    input, few distinct values, one heavy value, a constant, long-tailed and negative values,
+    infinities, signed zeros, a NaN, and one value next to a crowd of equal ones. Where infinities
+    leave NaN edges below finite ones, searchsorted has no answer of its own: there the row-major
+    and the feature-major binning must agree."""
+    import torch
+
+    from packboost_amd.data import quantile_bin_device
+
+    rng = np.random.default_rng(n + nb)
+    z = rng.standard_normal(n).astype(np.float32)
+    cols = [z, np.sort(z), np.sort(z)[::-1], np.round(z), np.where(rng.random(n) < 0.9, np.float32(0.25), z),
+            np.full(n, -7.5), np.exp(6 * z), -np.exp(-8 * z), np.where(rng.random(n) < 0.01, np.inf, z),
+            np.where(rng.random(n) < 0.4, -np.inf, z), np.where(rng.random(n) < 0.5, -0.0, 0.0),
+            np.where(np.arange(n) == n // 2, np.nan, z), np.where(np.arange(n) == n - 1, 1.0, 2.0), z * 1e-41]
+    X = np.stack([c.astype(np.float32) for c in cols], axis=1)
+    with np.errstate(invalid="ignore"):
+        want_b, want_e = _host_bins(X, nb)
+        ascends = np.array([np.array_equal(np.sort(e), e, equal_nan=True) for e in want_e.T])
+        got = []
+        for x in (X, torch.from_numpy(np.asfortranarray(X)).cuda()):
+            bins_fm, edges = quantile_bin_device(x, nb, torch.device("cuda"), chunk_features=9)
+            one_nan = [np.where(np.isnan(e), np.float32(np.nan), e) for e in (edges, want_e)]  # inf - inf: any sign
+            assert_edges_equal(*one_nan, f"n={n} nb={nb}")
+            got.append(bins_fm[:, :n].cpu().numpy().T)
+            np.testing.assert_array_equal(got[-1][:, ascends], want_b[:, ascends])
+    np.testing.assert_array_equal(got[0], got[1])
