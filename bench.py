@@ -483,12 +483,12 @@ def main() -> int:
     # Untimed for `value`: the same rounds with the per-round train era correlation that
     # PackBoost.fit logs (pb_era_corr on a side stream, read back each round), the reference's
     # log_metrics outside its round_seconds span (booster.py:654-655).
-    from packboost_amd.booster import _era_corr_device
+    from packboost_amd.booster import _corr_scratch, _era_corr_device
 
     fit = DeviceFit(bins, N, y, off, cfg)
     side = torch.cuda.Stream()
     era_off_dev = torch.from_numpy(np.asarray(off, dtype=np.int32)).cuda()
-    corr_scratch = torch.empty(len(off), dtype=torch.float64, device="cuda")
+    corr_scratch = _corr_scratch(N, len(off) - 1, torch.device("cuda"))
     rng_m = torch.Generator().manual_seed(42)
     corr = float("nan")
 

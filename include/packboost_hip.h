@@ -361,6 +361,13 @@ int pb_apply_bins(const float* xt_dev, int64_t n, int64_t ld_x, int32_t F, const
 int pb_era_corr(const float* y_dev, const float* preds_dev, const int32_t* era_off_dev,
                 int32_t num_eras, double* era_corr_dev, double* out_dev, void* stream);
 
+/* pb_era_corr of rows [0, n) (n = era_off[num_eras] < 2^31), with long eras spread over many
+ * workgroups: the sums are taken per window of 4096 rows and joined, in a fixed order. work_dev:
+ * double [pb_era_corr_work_elems(n, num_eras)] (-1: bad n or num_eras). */
+int64_t pb_era_corr_work_elems(int64_t n, int32_t num_eras);
+int pb_era_corr_rows(const float* y_dev, const float* preds_dev, int64_t n, const int32_t* era_off_dev,
+                     int32_t num_eras, double* era_corr_dev, double* work_dev, double* out_dev, void* stream);
+
 /* ---- prediction --------------------------------------------------------------------- */
 /* Kernel 4 — batched pack prediction. Replaces predict_pack_cuda (frontier_cuda.cu:925-1068):
  * out[r] = tree_weight * sum_t value(leaf_t(r)) over the B trees of one packed forest
@@ -424,6 +431,13 @@ int pb_predict_bins(const uint8_t* bins_dev, int64_t N, int64_t ld, int32_t F,
                     const int32_t* left_dev, const int32_t* right_dev,
                     const float* value_dev, const uint8_t* is_leaf_dev, int32_t num_nodes,
                     float* out_dev, void* stream);
+
+/* A pack of B identical trees added to running predictions tree by tree (the eval loop of
+ * booster.py:604-655): preds[r] = preds[r] + float32(weight * value(leaf(r))), B times, one float32
+ * rounding per product and per add. nodes_dev: int32 [num_nodes][4] = feature (-1: leaf),
+ * threshold, left child (the right one follows it), bits of the float32 value; 16-byte aligned. */
+int pb_fold_tree(const uint8_t* bins_dev, int64_t N, int64_t ld, int32_t F, const int32_t* nodes_dev,
+                 int32_t num_nodes, int32_t B, float weight, float* preds_dev, void* stream);
 
 /* ---- row lists ---------------------------------------------------------------------- */
 /* The reference's CUDA backend takes the rows of each frontier node as per-era lists:

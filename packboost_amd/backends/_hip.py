@@ -38,6 +38,7 @@ EXPORTED_SYMBOLS = (
     "pb_rowlist_gather", "pb_best_thresholds", "pb_pick_sequential", "pb_set_segment_mode", "pb_rowlist_noalloc_max_segments",
     "pb_rowlist_partition_noalloc", "pb_transpose_bins", "pb_forest_takes_rows",
     "pb_forest_predict_rows", "pb_bin_rows", "pb_quantile_work_bytes", "pb_column_quantiles",
+    "pb_era_corr_work_elems", "pb_era_corr_rows", "pb_fold_tree",
 )
 
 
@@ -113,6 +114,9 @@ _SIGNATURES = {
     "pb_grow_round": (ctypes.c_int, [_VP, ctypes.POINTER(PbFitBuffers), _VP, _I32, _VP, _VP, _VP]),
     "pb_profile_enable": (ctypes.c_int, [_VP, _I32]),
     "pb_era_corr": (ctypes.c_int, [_VP, _VP, _VP, _I32, _VP, _VP, _VP]),
+    "pb_era_corr_work_elems": (_I64, [_I64, _I32]),
+    "pb_era_corr_rows": (ctypes.c_int, [_VP, _VP, _I64, _VP, _I32, _VP, _VP, _VP, _VP]),
+    "pb_fold_tree": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _I32, _F32, _VP, _VP]),
     "pb_forest_create": (ctypes.c_int, [_VP] * 7 + [_I32, _I32, _VP]),
     "pb_forest_predict": (ctypes.c_int, [_VP, _VP, _I64, _I64, _I32, _F32, _VP, _VP, _VP]),
     "pb_forest_takes_rows": (_I32, [_VP]),

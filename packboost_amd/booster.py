@@ -322,12 +322,14 @@ class PackBoost:
         self._fitter = fitter
         k = subset_size(cfg, F)
         era_off_dev = torch.from_numpy(np.asarray(offsets, dtype=np.int32)).to(device)
-        corr_scratch = torch.empty(E + 1, dtype=torch.float64, device=device)
         eval_states = self._prepare_eval(eval_sets, device)
         eval_every = _eval_every()
         # metrics and eval predictions run on a side stream so that the next round, already
         # enqueued on the fit's stream, keeps the GPU busy while the host builds trees
         side = torch.cuda.Stream(device)
+        scratch = [_corr_scratch(N, E, device)] + [_corr_scratch(st["n"], st["num_eras"], device)
+                                                   for st in eval_states]
+        corrs = torch.empty(len(scratch), dtype=torch.float64, device=device)
         truncated = False
         try:
             t0 = perf_counter()
@@ -365,9 +367,11 @@ class PackBoost:
                     if eval_states and eval_every > 0 and (
                             (round_idx + 1) % eval_every == 0 or round_idx + 1 == num_rounds):
                         self._update_eval(eval_states)
-                    train_corr = _era_corr_device(fitter.y, preds_after, era_off_dev, corr_scratch)
-                    eval_corr = {f"{st['name']}_corr": _era_corr_device(
-                        st["y"], st["preds"], st["era_off"], st["corr_scratch"]) for st in eval_states}
+                    _era_corr_enqueue(fitter.y[:N], preds_after, era_off_dev, scratch[0], corrs[:1])
+                    for i, st in enumerate(eval_states):
+                        _era_corr_enqueue(st["y"][:st["n"]], st["preds"], st["era_off"], scratch[i + 1], corrs[i + 1:i + 2])
+                    train_corr, *rest = corrs.tolist()  # the round's one wait for its metrics
+                    eval_corr = {f"{st['name']}_corr": c for st, c in zip(eval_states, rest)}
                 t1 = perf_counter()
                 round_time = t1 - t0
                 t0 = t1
@@ -471,6 +475,8 @@ class PackBoost:
             # rows era-major (metrics only: eval predictions never leave the fit)
             perm, offs = era_major_order(codes, E)
             yv = np.asarray(y_eval, dtype=np.float32).reshape(-1)
+            if yv.shape[0] < n:
+                raise ValueError(f"eval set '{name}': X and y row mismatch")
             if perm is not None:
                 yv = yv[perm]
             edges = None if self.config.prebinned else self._binner.bin_edges
@@ -479,7 +485,6 @@ class PackBoost:
                 "name": name, "bins_fm": bins_fm, "n": n,
                 "y": torch.from_numpy(np.ascontiguousarray(yv)).to(device),
                 "era_off": torch.from_numpy(np.asarray(offs, dtype=np.int32)).to(device),
-                "corr_scratch": torch.empty(E + 1, dtype=torch.float64, device=device),
                 "num_eras": E,
                 "preds": torch.zeros(n, dtype=torch.float32, device=device),
                 "rounds_done": 0,
@@ -494,26 +499,29 @@ class PackBoost:
         # tree is walked once (pb_predict_bins) and its weighted value added B times. The host
         # work per eval is the new rounds only.
         B = int(self.config.pack_size)
-        w = torch.tensor(np.float32(self._tree_weight), dtype=torch.float32)
         lib = _hip.load()
+        trees: dict[int, torch.Tensor] = {}
         for st in states:
-            dev = st["preds"].device
-            wd = w.to(dev)
             while st["rounds_done"] < len(self._rounds):
-                a = self._rounds[st["rounds_done"]]
-                t = {k: torch.from_numpy(np.ascontiguousarray(np.asarray(a[k]), dtype=dt)).to(dev)
-                     for k, dt in (("feature", np.int32), ("threshold", np.int32), ("left", np.int32),
-                                   ("right", np.int32), ("value", np.float32), ("is_leaf", np.uint8))}
-                v = torch.empty(st["n"], dtype=torch.float32, device=dev)
-                _hip.check(lib.pb_predict_bins(
+                r = st["rounds_done"]
+                if r not in trees:
+                    trees[r] = torch.from_numpy(_tree_records(self._rounds[r])).to(st["preds"].device)
+                _hip.check(lib.pb_fold_tree(
                     st["bins_fm"].data_ptr(), st["n"], st["bins_fm"].shape[1], st["bins_fm"].shape[0],
-                    t["feature"].data_ptr(), t["threshold"].data_ptr(), t["left"].data_ptr(),
-                    t["right"].data_ptr(), t["value"].data_ptr(), t["is_leaf"].data_ptr(),
-                    int(t["value"].numel()), v.data_ptr(), _hip.stream_ptr()), "pb_predict_bins")
-                term = wd * v
-                for _ in range(B):
-                    st["preds"] = st["preds"] + term
+                    trees[r].data_ptr(), int(trees[r].shape[0]), B, float(np.float32(self._tree_weight)),
+                    st["preds"].data_ptr(), _hip.stream_ptr()), "pb_fold_tree")
                 st["rounds_done"] += 1
+
+
+def _tree_records(a: dict[str, np.ndarray]) -> np.ndarray:
+    """One tree's arrays as pb_fold_tree's node records, int32 [nodes, 4] (a split's right child
+    follows its left one, as TreeBuilder numbers them)."""
+    rec = np.empty((len(a["feature"]), 4), dtype=np.int32)
+    rec[:, 0] = np.where(a["is_leaf"], -1, a["feature"])
+    rec[:, 1] = a["threshold"]
+    rec[:, 2] = a["left"]
+    rec[:, 3] = np.asarray(a["value"]).astype(np.float32).view(np.int32)
+    return rec
 
 
 def pack_forest(rounds: Sequence[dict[str, np.ndarray]], pack_size: int,
@@ -551,12 +559,27 @@ def _eval_every() -> int:
         return 1
 
 
-def _era_corr_device(y: torch.Tensor, p: torch.Tensor, era_off: torch.Tensor,
-                     scratch: torch.Tensor) -> float:
-    """Mean over eras of the Pearson correlation of y and preds (booster.py:909-929) by the
-    pb_era_corr kernel on the current stream; rows are era-major, era_off int32 [E+1]."""
+def _corr_scratch(n: int, E: int, device: torch.device) -> torch.Tensor:
+    """Workspace of _era_corr_enqueue for n rows and E eras (double: per-era values, then window
+    sums)."""
+    elems = int(_hip.load().pb_era_corr_work_elems(n, E))
+    if elems < 0:
+        raise ValueError("era correlation needs fewer than 2^31 rows and at least one era")
+    return torch.empty(E + elems, dtype=torch.float64, device=device)
+
+
+def _era_corr_enqueue(y: torch.Tensor, p: torch.Tensor, era_off: torch.Tensor, scratch: torch.Tensor,
+                      out: torch.Tensor) -> None:
+    """out[0] = mean over eras of the Pearson correlation of y and preds (booster.py:909-929) by
+    pb_era_corr_rows on the current stream; rows are era-major, era_off int32 [E+1]."""
     E = int(era_off.numel()) - 1
-    lib = _hip.load()
-    _hip.check(lib.pb_era_corr(y.data_ptr(), p.data_ptr(), era_off.data_ptr(), E, scratch.data_ptr(),
-                               scratch.data_ptr() + 8 * E, _hip.stream_ptr()), "pb_era_corr")
-    return float(scratch[E].item())
+    _hip.check(_hip.load().pb_era_corr_rows(
+        y.data_ptr(), p.data_ptr(), int(y.numel()), era_off.data_ptr(), E, scratch.data_ptr(),
+        scratch.data_ptr() + 8 * E, out.data_ptr(), _hip.stream_ptr()), "pb_era_corr_rows")
+
+
+def _era_corr_device(y: torch.Tensor, p: torch.Tensor, era_off: torch.Tensor, scratch: torch.Tensor) -> float:
+    """_era_corr_enqueue's value, read back."""
+    out = torch.empty(1, dtype=torch.float64, device=y.device)
+    _era_corr_enqueue(y, p, era_off, scratch, out)
+    return float(out.item())

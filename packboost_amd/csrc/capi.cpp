@@ -1122,6 +1122,21 @@ int pb_era_corr(const float* y, const float* preds, const int32_t* era_off, int3
     return PB_OK;
 }
 
+int64_t pb_era_corr_work_elems(int64_t n, int32_t num_eras) {
+    if (n < 0 || n > INT32_MAX || num_eras < 1) return -1;
+    return 6 * pb::era_corr_slots(n, num_eras);
+}
+
+int pb_era_corr_rows(const float* y, const float* preds, int64_t n, const int32_t* era_off, int32_t num_eras,
+                     double* era_corr, double* work, double* out, void* stream) {
+    if (!y || !preds || !era_off || !era_corr || !work || !out)
+        return fail(PB_ERR_INVALID, "pb_era_corr_rows: null argument");
+    if (n < 0 || n > INT32_MAX || num_eras < 1) return fail(PB_ERR_INVALID, "pb_era_corr_rows: bad shape");
+    PB_HIP(pb::launch_era_corr_rows(y, preds, n, era_off, num_eras, era_corr, work, out, (hipStream_t)stream),
+           "era corr launch");
+    return PB_OK;
+}
+
 int pb_predict_forest(const uint8_t* bins, int64_t N, int64_t ld, int32_t F,
                       const int32_t* feature, const int32_t* threshold, const int32_t* left_abs,
                       const int32_t* right_abs, const float* value, const uint8_t* is_leaf,
@@ -1417,6 +1432,19 @@ int pb_predict_bins(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, const
     PB_HIP(pb::launch_predict_bins(bins, N, ld, F, feature, threshold, left, right, value, is_leaf,
                                    num_nodes, out, (hipStream_t)stream),
            "predict_bins launch");
+    return PB_OK;
+}
+
+int pb_fold_tree(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, const int32_t* nodes, int32_t num_nodes,
+                 int32_t B, float weight, float* preds, void* stream) {
+    if (N < 0 || ld < N || F < 1 || num_nodes < 1 || B < 0) return fail(PB_ERR_INVALID, "pb_fold_tree: bad shape");
+    if (N == 0 || B == 0) return PB_OK;
+    if (!bins || !nodes || !preds) return fail(PB_ERR_INVALID, "pb_fold_tree: null argument");
+    if (reinterpret_cast<uintptr_t>(nodes) & 15)
+        return fail(PB_ERR_INVALID, "pb_fold_tree: nodes must be 16-byte aligned");
+    PB_HIP(pb::launch_fold_tree(bins, N, ld, F, reinterpret_cast<const int4*>(nodes), num_nodes, B, weight, preds,
+                                (hipStream_t)stream),
+           "fold tree launch");
     return PB_OK;
 }
 

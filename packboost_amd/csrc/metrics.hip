@@ -2,11 +2,11 @@
 // predictions (PackBoost._era_correlation_np, booster.py:909-929). Rows are era-major, so era
 // e is the row range [era_off[e], era_off[e+1]).
 //
-// One workgroup per era, two passes in double (means, then centred sums), each reduced in a
-// fixed order (per-thread strided sums, then a fixed tree), so results are identical run to
-// run. An era counts when it has >= 2 rows, both population standard deviations exceed 1e-12
-// and the correlation is finite, as in the reference; the mean over counted eras is taken by
-// one thread in era order (NaN when none counts).
+// One workgroup per era (or, for long eras, per window of rows), two passes in double (means, then
+// centred sums), each reduced in a fixed order (per-thread strided sums, then a fixed tree), so
+// results are identical run to run. An era counts when it has >= 2 rows, both population standard
+// deviations exceed 1e-12 and the correlation is finite, as in the reference (the mean is NaN when
+// none counts).
 #include "pb_internal.h"
 
 namespace pb {
@@ -24,6 +24,16 @@ __device__ double block_sum(double v, double* sh) {
     double t = 0.0;
     for (int w = 0; w < kBlock / kWave; ++w) t += sh[w];
     return t;  // every thread holds the total
+}
+
+// The correlation of an era of n rows from its centred sums, NaN where the era does not count.
+__device__ __forceinline__ double corr_of(double n, double syy, double spp, double syp) {
+    const double nan = __longlong_as_double(0x7ff8000000000000ll);
+    if (!(n >= 2.0)) return nan;
+    const double sdy = sqrt(syy / n), sdp = sqrt(spp / n);
+    if (!(sdy > 1e-12 && sdp > 1e-12)) return nan;
+    const double v = (syp / n) / (sdy * sdp);
+    return isfinite(v) ? v : nan;
 }
 
 __global__ __launch_bounds__(kBlock) void era_corr_kernel(const float* __restrict__ y,
@@ -52,32 +62,142 @@ __global__ __launch_bounds__(kBlock) void era_corr_kernel(const float* __restric
     syy = block_sum(syy, sh);
     spp = block_sum(spp, sh);
     syp = block_sum(syp, sh);
-    if (threadIdx.x == 0) {
-        double c = __longlong_as_double(0x7ff8000000000000ll);  // NaN: era not counted
-        if (n >= 2) {
-            const double sdy = sqrt(syy / n), sdp = sqrt(spp / n);
-            if (sdy > 1e-12 && sdp > 1e-12) {
-                const double v = (syp / n) / (sdy * sdp);
-                if (isfinite(v)) c = v;
-            }
-        }
-        era_corr[e] = c;
-    }
+    if (threadIdx.x == 0) era_corr[e] = corr_of(n, syy, spp, syp);
 }
 
-__global__ void era_corr_mean_kernel(const double* __restrict__ era_corr, int32_t E,
-                                     double* __restrict__ out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s = 0.0;
-    int k = 0;
-    for (int e = 0; e < E; ++e) {
+// Mean over the counted eras by one workgroup in a fixed order (strided sums, then a tree): a single
+// thread walking them waited on a load per era (40 us for 574).
+__global__ __launch_bounds__(kBlock) void era_corr_mean_kernel(const double* __restrict__ era_corr, int32_t E,
+                                                           double* __restrict__ out) {
+    __shared__ double sh[kBlock / kWave];
+    double s = 0.0, k = 0.0;
+    for (int e = threadIdx.x; e < E; e += kBlock) {
         const double c = era_corr[e];
         if (!isnan(c)) {
             s += c;
-            ++k;
+            k += 1.0;
         }
     }
-    out[0] = k > 0 ? s / k : __longlong_as_double(0x7ff8000000000000ll);
+    s = block_sum(s, sh);
+    k = block_sum(k, sh);
+    if (threadIdx.x == 0) out[0] = k > 0.0 ? s / k : __longlong_as_double(0x7ff8000000000000ll);
+}
+
+// Eras of any length over many workgroups: one per window of kCorrWin consecutive rows, which keeps
+// its rows in registers and takes, for each era that overlaps it, the two passes of era_corr_kernel
+// over the overlap (means, then centred sums, in double). The pair (window w, era e) has slot w + e:
+// going up through the rows either w or e steps. era_corr_merge_kernel joins an era's windows.
+// One workgroup per era left a fit without eras (one era of 200k rows) 188 us per call; 12 + 4 us so.
+constexpr int kCorrRows = 16;  // rows per thread
+constexpr int kCorrWin = kBlock * kCorrRows;
+
+struct Moments {  // of one era's rows in one window
+    double n, my, mp, syy, spp, syp;
+};
+
+template <int K>
+__device__ __forceinline__ void block_sums(double (&v)[K], double (*sh)[4]) {
+    static_assert(K <= 4, "four sums at a time");
+#pragma unroll
+    for (int m = kWave / 2; m >= 1; m >>= 1)
+#pragma unroll
+        for (int k = 0; k < K; ++k) v[k] += __shfl_down(v[k], m);
+    __syncthreads();
+    if ((threadIdx.x & (kWave - 1)) == 0)
+#pragma unroll
+        for (int k = 0; k < K; ++k) sh[threadIdx.x / kWave][k] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        v[k] = 0.0;
+        for (int w = 0; w < kBlock / kWave; ++w) v[k] += sh[w][k];
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void era_corr_windows_kernel(const float* __restrict__ y, const float* __restrict__ p,
+                                                              int32_t n, const int32_t* __restrict__ era_off, int32_t E,
+                                                              Moments* __restrict__ slots) {
+    __shared__ double sh[kBlock / kWave][4];
+    const int w0 = blockIdx.x * kCorrWin;
+    const int w1 = min(w0 + kCorrWin, n);
+    float yv[kCorrRows], pv[kCorrRows];
+#pragma unroll
+    for (int i = 0; i < kCorrRows; ++i) {
+        const int r = w0 + i * kBlock + (int)threadIdx.x;
+        yv[i] = r < w1 ? y[r] : 0.0f;
+        pv[i] = r < w1 ? p[r] : 0.0f;
+    }
+    int lo = 0, hi = E - 1;  // the last era that starts at or before the window
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (era_off[mid] <= w0)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    for (int e = lo; e < E; ++e) {
+        const int r0 = max(era_off[e], w0), r1 = min(era_off[e + 1], w1);
+        if (era_off[e] >= w1) break;
+        if (r1 <= r0) continue;
+        double m[2] = {0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < kCorrRows; ++i) {
+            const int r = w0 + i * kBlock + (int)threadIdx.x;
+            if (r >= r0 && r < r1) {
+                m[0] += (double)yv[i];
+                m[1] += (double)pv[i];
+            }
+        }
+        block_sums(m, sh);
+        const double cnt = (double)(r1 - r0), my = m[0] / cnt, mp = m[1] / cnt;
+        double c[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < kCorrRows; ++i) {
+            const int r = w0 + i * kBlock + (int)threadIdx.x;
+            if (r >= r0 && r < r1) {
+                const double dy = (double)yv[i] - my, dp = (double)pv[i] - mp;
+                c[0] += dy * dy;
+                c[1] += dp * dp;
+                c[2] += dy * dp;
+            }
+        }
+        block_sums(c, sh);
+        if (threadIdx.x == 0) slots[(int64_t)blockIdx.x + e] = Moments{cnt, my, mp, c[0], c[1], c[2]};
+    }
+}
+
+// a joined with b (Chan, Golub and LeVeque's pairwise update)
+__device__ __forceinline__ void join(Moments& a, const Moments& b) {
+    const double n = a.n + b.n;
+    if (!(b.n > 0.0)) return;
+    const double dy = b.my - a.my, dp = b.mp - a.mp, f = b.n / n, g = a.n * f;
+    a.syy += b.syy + dy * dy * g;
+    a.spp += b.spp + dp * dp * g;
+    a.syp += b.syp + dy * dp * g;
+    a.my += dy * f;
+    a.mp += dp * f;
+    a.n = n;
+}
+
+// `lanes` (a power of two) lanes per era: each joins every lanes-th window of the era, then the lanes
+// are joined pairwise.
+__global__ __launch_bounds__(kBlock) void era_corr_merge_kernel(const Moments* __restrict__ slots,
+                                                            const int32_t* __restrict__ era_off, int32_t E,
+                                                            int32_t lanes, double* __restrict__ era_corr) {
+    const int t = blockIdx.x * kBlock + (int)threadIdx.x;
+    const int e = t / lanes, l = t & (lanes - 1);
+    Moments a{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (e < E) {
+        const int r0 = era_off[e], r1 = era_off[e + 1];
+        if (r1 > r0)
+            for (int w = r0 / kCorrWin + l; w <= (r1 - 1) / kCorrWin; w += lanes) join(a, slots[(int64_t)w + e]);
+    }
+    for (int m = 1; m < lanes; m <<= 1) {
+        const Moments b{__shfl_xor(a.n, m),   __shfl_xor(a.my, m),  __shfl_xor(a.mp, m),
+                        __shfl_xor(a.syy, m), __shfl_xor(a.spp, m), __shfl_xor(a.syp, m)};
+        join(a, b);
+    }
+    if (e < E && l == 0) era_corr[e] = corr_of(a.n, a.syy, a.spp, a.syp);
 }
 
 }  // namespace
@@ -87,7 +207,27 @@ hipError_t launch_era_corr(const float* y, const float* p, const int32_t* era_of
     hipLaunchKernelGGL(era_corr_kernel, dim3(E), dim3(kBlock), 0, s, y, p, era_off, era_corr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(era_corr_mean_kernel, dim3(1), dim3(64), 0, s, era_corr, E, out);
+    hipLaunchKernelGGL(era_corr_mean_kernel, dim3(1), dim3(kBlock), 0, s, era_corr, E, out);
+    return hipGetLastError();
+}
+
+int64_t era_corr_slots(int64_t n, int32_t E) { return (n + kCorrWin - 1) / kCorrWin + E; }
+
+hipError_t launch_era_corr_rows(const float* y, const float* p, int64_t n, const int32_t* era_off, int32_t E,
+                                double* era_corr, double* work, double* out, hipStream_t s) {
+    const int64_t wins = (n + kCorrWin - 1) / kCorrWin;
+    // up to two windows per era on average, a workgroup per era is as wide and skips the join (574
+    // eras of 4180 rows beside a running histogram: 32 us against 49 + 5)
+    if (n < (int64_t)E * (kCorrWin * 2)) return launch_era_corr(y, p, era_off, E, era_corr, out, s);
+    int32_t lanes = 1;
+    while (lanes < kWave && (int64_t)lanes * E < wins) lanes *= 2;
+    Moments* slots = reinterpret_cast<Moments*>(work);
+    hipLaunchKernelGGL(era_corr_windows_kernel, dim3((unsigned)wins), dim3(kBlock), 0, s, y, p, (int32_t)n, era_off, E,
+                       slots);
+    const int64_t threads = (int64_t)E * lanes;
+    hipLaunchKernelGGL(era_corr_merge_kernel, dim3((unsigned)((threads + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
+                       slots, era_off, E, lanes, era_corr);
+    hipLaunchKernelGGL(era_corr_mean_kernel, dim3(1), dim3(kBlock), 0, s, era_corr, E, out);
     return hipGetLastError();
 }
 

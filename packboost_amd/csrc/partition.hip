@@ -244,19 +244,23 @@ __global__ __launch_bounds__(kBlock) void round_begin_kernel(const float* __rest
     }
 }
 
-// One thread per era: the era's |grad| sum is at most the sum over the windows it overlaps;
-// sh_era[e] = era_grad_scale of that bound.
+// One wavefront per era: the era's |grad| sum is at most the sum over the windows it overlaps
+// (lanes stride over them, then a fixed tree); sh_era[e] = era_grad_scale of that bound.
 // Also flags the round (Frontier::reserved[kNonFinite]) when an era's |grad| bound is not finite:
 // a NaN or infinite gradient (or one whose window sum overflows float) has no fixed-point value.
 __global__ __launch_bounds__(kBlock) void era_scale_kernel(const int32_t* __restrict__ era_off, int32_t E,
                                                        const float* __restrict__ win_sum,
                                                        int32_t* __restrict__ sh_era, Frontier* st) {
-    const int e = blockIdx.x * kBlock + threadIdx.x;
-    if (e >= E) return;
+    const int e = blockIdx.x * (kBlock / kWave) + (int)threadIdx.x / kWave;
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    if (e >= E) return;  // whole wavefronts
     const int64_t r0 = era_off[e], r1 = era_off[e + 1];
     double b = 0.0;
     if (r1 > r0)
-        for (int64_t w = r0 / kGradWinRows; w <= (r1 - 1) / kGradWinRows; ++w) b += (double)win_sum[w];
+        for (int64_t w = r0 / kGradWinRows + lane; w <= (r1 - 1) / kGradWinRows; w += kWave) b += (double)win_sum[w];
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) b += __shfl_xor(b, m);
+    if (lane) return;
     if (!isfinite(b)) st->reserved[kNonFinite] = 1;
     sh_era[e] = era_grad_scale(b * (1.0 + 1.0 / 1024.0));
 }
@@ -358,7 +362,8 @@ hipError_t launch_round_begin(const float* preds, const float* y, float* grad, u
                            tnode, N, rows_padded, root_active, win_sum, st, cur_ids);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(era_scale_kernel, dim3((E + kBlock - 1) / kBlock), dim3(kBlock), 0, s, era_off,
+    constexpr int kEras = kBlock / kWave;
+    hipLaunchKernelGGL(era_scale_kernel, dim3((E + kEras - 1) / kEras), dim3(kBlock), 0, s, era_off,
                        E, win_sum, sh_era, st);
     return hipGetLastError();
 }

@@ -423,6 +423,13 @@ hipError_t launch_apply_bins(const float* xt, int64_t n, int64_t ld_x, int32_t F
                              const int64_t* perm, uint8_t* bins, int64_t ld_out, hipStream_t s);
 hipError_t launch_era_corr(const float* y, const float* p, const int32_t* era_off, int32_t E,
                            double* era_corr, double* out, hipStream_t s);
+hipError_t launch_fold_tree(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, const int4* nodes,
+                            int32_t num_nodes, int32_t B, float w, float* preds, hipStream_t s);
+// The same for rows [0, n) and eras of any length, over n / 4096 workgroups: work holds
+// 6 * era_corr_slots(n, E) doubles.
+int64_t era_corr_slots(int64_t n, int32_t E);
+hipError_t launch_era_corr_rows(const float* y, const float* p, int64_t n, const int32_t* era_off, int32_t E,
+                                double* era_corr, double* work, double* out, hipStream_t s);
 hipError_t launch_forest(const uint8_t* bins, int64_t N, int64_t ld, const int4* rec,
                          const int32_t* roots, int32_t T, int32_t depth, float tree_weight,
                          float* out, int32_t* leaf, int32_t group, int32_t max_grid,

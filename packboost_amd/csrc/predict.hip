@@ -84,6 +84,43 @@ __global__ __launch_bounds__(kBlock) void predict_bins_kernel(
     }
 }
 
+// preds[r] = preds[r] + float32(w * leaf value), B times, one float32 rounding per product and per
+// add: a pack of B identical trees added tree by tree. The tree's 16-byte records (feature or -1,
+// threshold, left child with the right one next to it, value bits) are staged in LDS while they
+// fit: a lane's walk then waits on its bins alone. One launch replaces the walk, the product and
+// B separate adds over the rows.
+constexpr int kFoldLdsNodes = 1024;
+
+__global__ __launch_bounds__(kBlock) void fold_tree_kernel(const uint8_t* __restrict__ bins, int64_t N, int64_t ld,
+                                                       int32_t F, const int4* __restrict__ nodes, int32_t num_nodes,
+                                                       int32_t B, float w, float* __restrict__ preds) {
+    __shared__ int4 s_node[kFoldLdsNodes];
+    const bool in_lds = num_nodes <= kFoldLdsNodes;
+    if (in_lds) {
+        for (int i = threadIdx.x; i < num_nodes; i += kBlock) s_node[i] = nodes[i];
+        __syncthreads();
+    }
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < N; r += stride) {
+        float p = preds[r];
+        int4 q = in_lds ? s_node[0] : nodes[0];
+        float v = 0.0f;
+        for (int it = 0; it < num_nodes; ++it) {
+            if (q.x < 0) {
+                v = __int_as_float(q.w);
+                break;
+            }
+            if (q.x >= F) break;
+            const int32_t next = q.z + ((int32_t)bins[(int64_t)q.x * ld + r] <= q.y ? 0 : 1);
+            if (next < 0 || next >= num_nodes) break;
+            q = in_lds ? s_node[next] : nodes[next];
+        }
+        const float term = w * v;
+        for (int b = 0; b < B; ++b) p = p + term;
+        preds[r] = p;
+    }
+}
+
 // Compiled forest: one 16-byte record per node {feature | threshold << 24, left, right,
 // value bits}; a leaf has feature field 0xFFFFFF. A lane walks kTreeGroup trees at once, all
 // one level per step, so their record and bin loads overlap; the leaf values are then added
@@ -483,6 +520,13 @@ hipError_t launch_predict_pack(const uint8_t* bins, int64_t N, int64_t ld, int32
     hipLaunchKernelGGL(predict_pack_kernel, dim3(grid_rows(N)), dim3(kBlock), 0, s, bins, N, ld,
                        F, feature, threshold, left_abs, right_abs, value, is_leaf, offsets, B,
                        total_nodes, tree_weight, sequential, out, leaf);
+    return hipGetLastError();
+}
+
+hipError_t launch_fold_tree(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, const int4* nodes,
+                            int32_t num_nodes, int32_t B, float w, float* preds, hipStream_t s) {
+    hipLaunchKernelGGL(fold_tree_kernel, dim3(grid_rows(N)), dim3(kBlock), 0, s, bins, N, ld, F, nodes, num_nodes, B,
+                       w, preds);
     return hipGetLastError();
 }
 

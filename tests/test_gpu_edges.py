@@ -278,3 +278,25 @@ def test_nonfinite_gradients_stop_the_fit(hip, monkeypatch, case):
     y_ok = np.nan_to_num(y, nan=0.0, posinf=0.0)
     model2 = PackBoost(PackBoostConfig(pack_size=2, learning_rate=0.1, **kw)).fit(X, y_ok, era, num_rounds=2)
     assert np.all(np.isfinite(model2.predict(X[:100])))
+
+
+@pytest.mark.parametrize("nb", [2, 3, 5, 16, 17, 32, 33, 63, 64, 65, 128, 255])
+def test_split_era_bins(hip, monkeypatch, nb):
+    """Split eras at every lane grouping of the finalising pass: the planes equal those of the same
+    eras built whole, bit for bit (both are exact sums rounded once)."""
+    sizes, U, F = (3000, 900, 5001), 3, 4
+    p = make_problem(nb, int(sum(sizes)), F, len(sizes), nb, U, ragged=False)
+    p["era_off"] = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    p["era"] = np.repeat(np.arange(len(sizes)), sizes)
+    feats = np.arange(F, dtype=np.int32)
+    planes = []
+    for rows in ("16384", "700"):
+        monkeypatch.setenv("PB_HIST_SEG_ROWS", rows)
+        g = GpuDepth(hip, p, F, msl=1, layout="u8")
+        try:
+            g.hist(feats)
+            planes.append(g.planes())
+        finally:
+            g.close()
+    np.testing.assert_array_equal(planes[0][0], planes[1][0])
+    np.testing.assert_array_equal(planes[0][1], planes[1][1])

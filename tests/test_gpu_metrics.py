@@ -92,3 +92,65 @@ def test_fit_round_metrics(hip):
     # PackBoost.predict (the compiled forest's double sums, rounded once) within 1e-5 of it
     np.testing.assert_allclose(model.predict(X2), p_eval, rtol=0, atol=1e-5)
     assert all(np.isfinite(r["train_corr"]) for r in model.round_metrics)
+
+
+@pytest.mark.parametrize("sizes", [
+    [1], [4096], [4097], [20_000], [4095, 1, 0, 4096, 0, 50_000], [0, 0, 70_000, 2, 0, 1, 12_289, 0],
+    [400_000] + [3] * 40 + [50_000], [9000] * 70], ids=str)
+def test_era_corr_rows(hip, sizes):
+    """pb_era_corr_rows (long eras over many workgroups: window edges, windows of several eras,
+    empty, single-row and constant eras) against float64 NumPy and pb_era_corr, within 1e-9."""
+    import torch
+
+    from packboost_amd.booster import _corr_scratch, _era_corr_enqueue
+
+    E, N = len(sizes), int(sum(sizes))
+    rng = np.random.default_rng(N)
+    era = np.repeat(np.arange(E), sizes)
+    y = (3 + rng.standard_normal(N)).astype(np.float32)
+    p = (0.3 * y + rng.standard_normal(N) - 7).astype(np.float32)
+    if E > 4:
+        p[era == 3] = -1.5  # constant: skipped
+    dev = torch.device("cuda")
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)).to(dev)
+    yd, pd_ = torch.from_numpy(y).to(dev), torch.from_numpy(p).to(dev)
+    scratch = _corr_scratch(N, E, dev)
+    out, old = torch.empty(1, dtype=torch.float64, device=dev), torch.empty(E + 1, dtype=torch.float64, device=dev)
+    _era_corr_enqueue(yd, pd_, off, scratch, out)
+    hip.check(hip.load().pb_era_corr(yd.data_ptr(), pd_.data_ptr(), off.data_ptr(), E, old.data_ptr(),
+                                     old.data_ptr() + 8 * E, hip.stream_ptr()), "pb_era_corr")
+    got, was = scratch[:E].cpu().numpy(), old.cpu().numpy()
+    for e in range(E):
+        want = era_corr_np(np.zeros(sizes[e]), y[era == e], p[era == e])
+        np.testing.assert_allclose([got[e], was[e]], [want, want], rtol=0, atol=1e-9)
+    np.testing.assert_allclose([out.item(), was[E]], [era_corr_np(era, y, p)] * 2, rtol=0, atol=1e-9)
+
+
+@pytest.mark.parametrize("depth,B", [(0, 3), (1, 1), (6, 8), (9, 2), (10, 5)])
+def test_fold_tree(hip, depth, B):
+    """pb_fold_tree (records in LDS up to 1024 nodes, in memory above) against pb_predict_bins and
+    B separate float32 adds: the same roundings, so equal bit for bit."""
+    import torch
+
+    from packboost_amd.booster import _to_column_major, _tree_records
+    from tests.test_gpu_forest import _forest
+
+    dev = torch.device("cuda")
+    N, F = 3001, 40
+    a = _forest(depth, 2, 1, depth, F, ragged=True, max_thr=30)[1]
+    bins = _to_column_major(torch.randint(0, 32, (N, F), dtype=torch.uint8, device=dev), dev)
+    lib, v = hip.load(), torch.empty(N, device=dev)
+    t = {k: torch.from_numpy(np.ascontiguousarray(a[k]).astype(d)).to(dev) for k, d in (
+        ("feature", np.int32), ("threshold", np.int32), ("left", np.int32), ("right", np.int32),
+        ("value", np.float32), ("is_leaf", np.uint8))}
+    hip.check(lib.pb_predict_bins(bins.data_ptr(), N, bins.shape[1], F, *(t[k].data_ptr() for k in t),
+                                  len(a["value"]), v.data_ptr(), hip.stream_ptr()), "pb_predict_bins")
+    want = torch.randn(N, device=dev)
+    got = want.clone()
+    term = torch.tensor(0.1, device=dev) * v
+    for _ in range(B):
+        want = want + term
+    rec = torch.from_numpy(_tree_records(a)).to(dev)
+    hip.check(lib.pb_fold_tree(bins.data_ptr(), N, bins.shape[1], F, rec.data_ptr(), len(a["value"]), B,
+                               float(np.float32(0.1)), got.data_ptr(), hip.stream_ptr()), "pb_fold_tree")
+    assert torch.equal(got, want)
