@@ -48,17 +48,16 @@ def cuda_available() -> bool:
     return _hip.device_available()
 
 
-def _u8_fm(bins: torch.Tensor) -> torch.Tensor:
-    """Feature-major [F, N] int8/uint8 -> contiguous uint8 [F, ld] with ld % 16 == 0."""
+def _u8_fm(bins: torch.Tensor) -> tuple[torch.Tensor, int]:
+    """Feature-major [F, N] bins as uint8 with adjacent rows, and their column stride: int8 / uint8
+    bins are taken as they lie, others are converted."""
     if bins.dim() != 2:
         raise ValueError("bins must be 2-D feature-major [F, N]")
-    F, N = bins.shape
-    ld = (int(N) + 15) // 16 * 16
-    if bins.dtype == torch.uint8 and ld == N and bins.is_contiguous():
-        return bins
-    out = torch.zeros((int(F), ld), dtype=torch.uint8, device=bins.device)
-    out[:, :N] = bins.view(torch.uint8) if bins.dtype == torch.int8 else bins.to(torch.uint8)
-    return out
+    N = int(bins.shape[1])
+    b = bins.view(torch.uint8) if bins.dtype == torch.int8 else bins.to(torch.uint8)
+    if (N > 1 and b.stride(1) != 1) or b.stride(0) < N:
+        b = b.contiguous()
+    return b, max(int(b.stride(0)), N)
 
 
 def predict_bins_cuda(bins_fm: torch.Tensor, feature: torch.Tensor, threshold: torch.Tensor,
@@ -67,13 +66,13 @@ def predict_bins_cuda(bins_fm: torch.Tensor, feature: torch.Tensor, threshold: t
     """One tree over feature-major bins (frontier_cuda.cu:853-920): float32 [N] leaf values."""
     lib = _hip.load()
     F, N = bins_fm.shape
-    b = _u8_fm(bins_fm)
+    b, ld = _u8_fm(bins_fm)
     dev = b.device
     cast = lambda t, dt: t.to(device=dev, dtype=dt).contiguous()  # noqa: E731
     f, t, l, r = (cast(x, torch.int32) for x in (feature, threshold, left, right))
     v, lf = cast(value, torch.float32), cast(is_leaf, torch.uint8)
     out = torch.empty(int(N), dtype=torch.float32, device=dev)
-    _hip.check(lib.pb_predict_bins(b.data_ptr(), int(N), b.shape[1], int(F), f.data_ptr(),
+    _hip.check(lib.pb_predict_bins(b.data_ptr(), int(N), ld, int(F), f.data_ptr(),
                                    t.data_ptr(), l.data_ptr(), r.data_ptr(), v.data_ptr(),
                                    lf.data_ptr(), int(f.numel()), out.data_ptr(),
                                    _hip.stream_ptr()), "pb_predict_bins")
@@ -88,13 +87,13 @@ def predict_pack_cuda(bins_fm: torch.Tensor, feature: torch.Tensor, threshold: t
     F, N = bins_fm.shape
     if int(N) == 0:
         return torch.empty(0, dtype=torch.float32, device=bins_fm.device)
-    b = _u8_fm(bins_fm)
+    b, ld = _u8_fm(bins_fm)
     dev = b.device
     cast = lambda t, dt: t.to(device=dev, dtype=dt).contiguous()  # noqa: E731
     f, t, l, r, o = (cast(x, torch.int32) for x in (feature, threshold, left_abs, right_abs, offsets))
     v, lf = cast(value, torch.float32), cast(is_leaf, torch.uint8)
     out = torch.empty(int(N), dtype=torch.float32, device=dev)
-    _hip.check(lib.pb_predict_pack(b.data_ptr(), int(N), b.shape[1], int(F), f.data_ptr(),
+    _hip.check(lib.pb_predict_pack(b.data_ptr(), int(N), ld, int(F), f.data_ptr(),
                                    t.data_ptr(), l.data_ptr(), r.data_ptr(), v.data_ptr(),
                                    lf.data_ptr(), o.data_ptr(), int(o.numel() - 1), int(f.numel()),
                                    float(tree_weight), out.data_ptr(), None, _hip.stream_ptr()),

@@ -70,6 +70,79 @@ __global__ __launch_bounds__(kBlock) void predict_pack_kernel(
     }
 }
 
+// predict_pack_kernel for forests of up to kPackNodes nodes: the nodes sit in LDS as 16-byte records
+// (feature, or -1 for a leaf with its value bits in the next word; threshold; children) and a lane
+// walks 8 trees a level at a time, so that their bin loads are in flight together. The one-tree
+// walk waited on a node and a bin in turn, 48 times in a row for 8 trees of depth 6:
+// 188 us for 600k rows, 54 us so (about the bytes of the columns it reads at the copy rate).
+constexpr int kPackNodes = 2048;
+constexpr int kPackTrees = 8;
+
+__global__ __launch_bounds__(kBlock) void predict_pack_lds_kernel(
+    const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F, const int32_t* __restrict__ feature,
+    const int32_t* __restrict__ threshold, const int32_t* __restrict__ left_abs, const int32_t* __restrict__ right_abs,
+    const float* __restrict__ value, const uint8_t* __restrict__ is_leaf, const int32_t* __restrict__ offsets, int32_t B,
+    int32_t total_nodes, float tree_weight, int32_t sequential, float* __restrict__ out, int32_t* __restrict__ leaf) {
+    __shared__ int4 s_node[kPackNodes];
+    for (int i = threadIdx.x; i < total_nodes; i += kBlock) {
+        const int f = feature[i];
+        // a split on a feature outside [0, F) ends the walk: -2
+        s_node[i] = is_leaf[i] ? make_int4(-1, __float_as_int(value[i]), 0, 0)
+                               : make_int4(f >= 0 && f < F ? f : -2, threshold[i], left_abs[i], right_abs[i]);
+    }
+    __syncthreads();
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < N; r += stride) {
+        float s = 0.0f;
+        for (int t0 = 0; t0 < B; t0 += kPackTrees) {
+            int32_t node[kPackTrees], lo[kPackTrees], hi[kPackTrees], lf[kPackTrees];
+            float v[kPackTrees];
+            int32_t steps = 0;
+#pragma unroll
+            for (int j = 0; j < kPackTrees; ++j) {
+                // a tree's span, clamped to the node arrays (offsets come from the caller)
+                const int t = min(t0 + j, B - 1);
+                lo[j] = min(max(offsets[t], 0), total_nodes);
+                hi[j] = min(max(offsets[t + 1], lo[j]), total_nodes);
+                node[j] = t0 + j < B && lo[j] < hi[j] ? lo[j] : -1;  // -1: done
+                v[j] = 0.0f;
+                lf[j] = -1;
+                steps = max(steps, hi[j] - lo[j]);
+            }
+            for (int it = 0; it < steps; ++it) {
+                int4 q[kPackTrees];
+                int32_t bin[kPackTrees];
+#pragma unroll
+                for (int j = 0; j < kPackTrees; ++j) q[j] = s_node[max(node[j], 0)];
+#pragma unroll
+                for (int j = 0; j < kPackTrees; ++j)  // in bounds whatever the record
+                    bin[j] = bins[(int64_t)max(q[j].x, 0) * ld + r];
+                bool live = false;
+#pragma unroll
+                for (int j = 0; j < kPackTrees; ++j) {
+                    if (node[j] < 0) continue;
+                    const int32_t next = bin[j] <= q[j].y ? q[j].z : q[j].w;
+                    if (q[j].x == -1) {
+                        v[j] = __int_as_float(q[j].y);
+                        lf[j] = node[j];
+                    }
+                    const bool on = q[j].x >= 0 && next >= lo[j] && next < hi[j] && it + 1 < hi[j] - lo[j];
+                    node[j] = on ? next : -1;
+                    live |= on;
+                }
+                if (!live) break;
+            }
+#pragma unroll
+            for (int j = 0; j < kPackTrees; ++j) {
+                if (t0 + j >= B) continue;
+                s = sequential ? (s + tree_weight * v[j]) : (s + v[j]);
+                if (leaf) leaf[(int64_t)(t0 + j) * N + r] = lf[j];
+            }
+        }
+        out[r] = sequential ? s : tree_weight * s;
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void predict_bins_kernel(
     const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F,
     const int32_t* __restrict__ feature, const int32_t* __restrict__ threshold,
@@ -517,6 +590,14 @@ hipError_t launch_predict_pack(const uint8_t* bins, int64_t N, int64_t ld, int32
                                const int32_t* offsets, int32_t B, int32_t total_nodes,
                                float tree_weight, int32_t sequential, float* out, int32_t* leaf,
                                hipStream_t s) {
+    // the LDS walk while the forest fits its records (about 16 depth-6 trees); a longer forest's nodes
+    // are read where they lie
+    if (total_nodes > 0 && total_nodes <= kPackNodes) {
+        hipLaunchKernelGGL(predict_pack_lds_kernel, dim3(grid_rows(N)), dim3(kBlock), 0, s, bins, N, ld, F, feature,
+                           threshold, left_abs, right_abs, value, is_leaf, offsets, B, total_nodes, tree_weight,
+                           sequential, out, leaf);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(predict_pack_kernel, dim3(grid_rows(N)), dim3(kBlock), 0, s, bins, N, ld,
                        F, feature, threshold, left_abs, right_abs, value, is_leaf, offsets, B,
                        total_nodes, tree_weight, sequential, out, leaf);

@@ -89,3 +89,31 @@ def test_predict_pack_empty_and_errors(hip):
             bad["right_abs"][0] = val
         got = predict_pack_cuda(bins, *(bad[k] for k in args), bad["offsets"], 1.0)
         np.testing.assert_array_equal(got.cpu().numpy(), second_only.cpu().numpy())
+
+
+@pytest.mark.parametrize("B,D", [(1, 0), (7, 3), (8, 6), (9, 6), (16, 6), (17, 6), (3, 9), (2, 10)])
+@pytest.mark.parametrize("view", ["odd", "slice", "columns", "int64"])
+def test_pack_shapes(hip, B, D, view):
+    """The LDS walk (up to 2048 nodes) and the walk in memory (17 trees of depth 6, 2 of depth 10),
+    part-filled groups of trees, odd strides, views and converted inputs: each tree alone through
+    predict_bins_cuda, added in tree order in float32, gives the same sum bit for bit."""
+    import torch
+
+    from packboost_amd.backends import predict_bins_cuda, predict_pack_cuda
+    from packboost_amd.booster import pack_forest
+
+    dev = torch.device("cuda")
+    N, F = 1003, 50
+    rounds = _forest(31 * B + D, B, 1, D, F, ragged=True, max_thr=20)
+    wide = torch.randint(0, 22, (F, N + 9), dtype=torch.uint8, device=dev)
+    bins = {"odd": wide[:, :N].contiguous(), "slice": wide[:, 5:5 + N], "int64": wide[:, :N].long(),
+            "columns": wide[:, :N].t().contiguous().t()}[view]
+    f = pack_forest(rounds, 1, dev)
+    args = ("feature", "threshold", "left_abs", "right_abs", "value", "is_leaf", "offsets")
+    got = predict_pack_cuda(bins, *(f[k] for k in args), 0.3)
+    want = torch.zeros(N, device=dev)
+    for a in rounds:
+        t = {k: torch.from_numpy(np.ascontiguousarray(a[k])).to(dev) for k in
+             ("feature", "threshold", "left", "right", "value", "is_leaf")}
+        want = want + predict_bins_cuda(wide[:, 5:5 + N] if view == "slice" else wide[:, :N], *t.values())
+    assert torch.equal(got, torch.tensor(0.3, device=dev) * want)
