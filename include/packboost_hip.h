@@ -498,6 +498,23 @@ int pb_rowlist_gather(const uint8_t* bins_dev, int64_t N, int64_t ld, int32_t F,
                       int32_t E, uint8_t* out_bins_dev, int64_t out_ld, float* out_values_dev,
                       uint16_t* out_slot_dev, int32_t* era_off_dev, int32_t* work_dev, void* stream);
 
+/* What the adapter of find_best_splits_batched_cuda must know of its inputs before it scores them,
+ * in one launch (the caller clears *out_dev): whether hess_dev [n_hess] holds anything but 1
+ * (bad_hess), a weight of an era without rows is not 0 (stray_weight), some era has rows (counted)
+ * and a weight other than 1 (not_unit), a drawn feature id lies outside [0, F) (bad_feature), a bin
+ * of a drawn column is >= limit (bin_over); the least and greatest weight - rows over eras with
+ * rows (alpha_lo, alpha_hi: -inf, inf with a NaN weight), and the listed rows of all nodes. bins
+ * uint8 [F][ld] (any alignment), weights float32 [M][E], node_era_splits int32 [M][E + 1]. */
+typedef struct pb_rowlist_facts {
+    int32_t bad_hess, stray_weight, counted, not_unit, bad_feature, bin_over, reserved[2];
+    double alpha_lo, alpha_hi;
+    int64_t rows, reserved2;
+} pb_rowlist_facts;
+int pb_rowlist_facts_get(const uint8_t* bins_dev, int64_t N, int64_t ld, int32_t F, const int32_t* feats_dev,
+                         int32_t K, const float* hess_dev, int64_t n_hess, const float* weights_dev,
+                         const int32_t* node_era_splits_dev, int32_t M, int32_t E, int32_t limit,
+                         pb_rowlist_facts* out_dev, void* stream);
+
 /* The per-(node, feature) pick of find_best_splits_batched_cuda (frontier_cuda.cu:537-560)
  * over candidate records cand_dev [M][K][T] (pb_des_score's cand_all_dev, thresholds in
  * order): the best valid score wins; within 1e-12 of it the larger left count, then the

@@ -39,6 +39,7 @@ EXPORTED_SYMBOLS = (
     "pb_rowlist_partition_noalloc", "pb_transpose_bins", "pb_forest_takes_rows",
     "pb_forest_predict_rows", "pb_bin_rows", "pb_quantile_work_bytes", "pb_column_quantiles",
     "pb_era_corr_work_elems", "pb_era_corr_rows", "pb_fold_tree",
+    "pb_rowlist_facts_get",
 )
 
 
@@ -87,6 +88,12 @@ CANDIDATE_DTYPE = np.dtype([
     ("score", "<f4"), ("left_total", "<i4"), ("left_grad", "<f4"), ("feature", "<i4"),
     ("threshold", "<i4"), ("valid", "<i4"), ("reserved", "<i4", (2,)),
 ])
+FACTS_DTYPE = np.dtype([
+    ("bad_hess", "<i4"), ("stray_weight", "<i4"), ("counted", "<i4"), ("not_unit", "<i4"), ("bad_feature", "<i4"),
+    ("bin_over", "<i4"), ("reserved", "<i4", (2,)), ("alpha_lo", "<f8"), ("alpha_hi", "<f8"), ("rows", "<i8"),
+    ("reserved2", "<i8"),
+])
+assert FACTS_DTYPE.itemsize == 64
 assert DECISION_DTYPE.itemsize == 64 and CANDIDATE_DTYPE.itemsize == 32
 assert HEADER_DTYPE.itemsize == 96
 
@@ -145,6 +152,8 @@ _SIGNATURES = {
                                             _VP, _VP, _VP, _I64, _VP, _VP, _VP, _VP]),
     "pb_rowlist_gather": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _VP, _VP, _I64, _VP, _VP,
                                          _I32, _I32, _I32, _VP, _I64, _VP, _VP, _VP, _VP, _VP]),
+    "pb_rowlist_facts_get": (ctypes.c_int, [_VP, _I64, _I64, _I32, _VP, _I32, _VP, _I64, _VP, _VP, _I32, _I32, _I32,
+                                            _VP, _VP]),
     "pb_best_thresholds": (ctypes.c_int, [_VP, _I32, _I32, _I32, _VP, _VP, _VP, _VP, _VP, _VP]),
     "pb_pick_sequential": (ctypes.c_int, [_VP, _I32, _I32, _I32, _VP, _VP, _VP]),
     "pb_set_segment_mode": (ctypes.c_int, [_VP, _I32, _I32]),

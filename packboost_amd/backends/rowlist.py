@@ -49,12 +49,34 @@ def _era_alpha(era_weights: torch.Tensor, counts: torch.Tensor) -> float:
     return float(alpha[0])
 
 
+def _era_alpha_of(facts: np.ndarray) -> float:
+    """_era_alpha from the device's facts."""
+    if facts["stray_weight"]:
+        raise RuntimeError("era_weights must be 0 for eras without rows")
+    if not facts["counted"] or not facts["not_unit"]:
+        return 0.0
+    if facts["alpha_lo"] != facts["alpha_hi"] or not facts["alpha_lo"] > 0.0:
+        raise RuntimeError("era_weights are not count + era_alpha for one era_alpha > 0")
+    return float(facts["alpha_lo"])
+
+
 _STATUS = ("a (node, era) segment lies outside rows_index", "a row id lies outside [0, N)",
            "a feature id lies outside [0, F)", "an output would pass its capacity")
 
 
-def _check_status(work: torch.Tensor, what: str) -> None:
-    st = work[:4].cpu().tolist()
+def _facts(lib, b_fm, F, N, ld, fid, K, hess, weights, nes, M, E, limit) -> np.ndarray:
+    """pb_rowlist_facts of the call's inputs: one launch and one wait."""
+    dev = b_fm.device
+    out = torch.zeros(_hip.FACTS_DTYPE.itemsize, dtype=torch.uint8, device=dev)
+    h = hess.to(device=dev, dtype=torch.float32).contiguous()
+    _hip.check(lib.pb_rowlist_facts_get(b_fm.data_ptr(), N, ld, F, fid.data_ptr(), K, h.data_ptr(), int(h.numel()),
+                                        weights.data_ptr(), nes.data_ptr(), M, E, limit, out.data_ptr(),
+                                        _hip.stream_ptr()), "pb_rowlist_facts_get")
+    return np.frombuffer(out.cpu().numpy().tobytes(), dtype=_hip.FACTS_DTYPE)[0]
+
+
+def _check_status(work: torch.Tensor | np.ndarray, what: str) -> None:
+    st = (work if isinstance(work, np.ndarray) else work[:4].cpu().numpy()).tolist()
     bad = [msg for flag, msg in zip(st, _STATUS) if flag]
     if bad:
         raise RuntimeError(f"{what}: " + "; ".join(bad))
@@ -89,8 +111,6 @@ def find_best_splits_batched_rowlist(bins, grad, hess, rows_index, node_row_spli
     nb = int(max_bins)
     if not 2 <= nb <= 255:
         raise ValueError("max_bins must lie in [2, 255]")
-    if bool((hess.to(torch.float32) != 1.0).any()):
-        raise RuntimeError("HIP backend supports squared loss only (hess == 1)")
     b_fm, F, N, ld_in = _bins_fm(bins)
     rows = _i32(rows_index, dev)
     nrs = _i32(node_row_splits, dev)
@@ -98,31 +118,36 @@ def find_best_splits_batched_rowlist(bins, grad, hess, rows_index, node_row_spli
     E = int(nes.shape[1]) - 1
     if E < 1:
         raise ValueError("node_era_splits must have at least 2 columns")
-    counts = nes[:, 1:] - nes[:, :-1]  # [M, E]
-    alpha = _era_alpha(era_weights, counts)
+    if int(nes.shape[0]) < M:
+        raise ValueError("node_era_splits needs one row per node")
     K = int(feature_ids.numel())
     fid = _i32(feature_ids, dev)
-    vals = grad.to(device=dev, dtype=torch.float32).contiguous()
     R = int(rows.numel())
+    # float32 weights of the lists' shape are looked at on the device with the rest; others keep
+    # their own precision on the host
+    w_dev = era_weights.to(device=dev).contiguous() if (
+        era_weights.dtype == torch.float32 and tuple(era_weights.shape) == (M, E) and int(nes.shape[0]) == M) else None
+    facts = _facts(lib, b_fm, F, N, ld_in, fid, K, hess,
+                   torch.zeros((M, E), dtype=torch.float32, device=dev) if w_dev is None else w_dev, nes, M, E, nb)
+    if facts["bad_hess"]:
+        raise RuntimeError("HIP backend supports squared loss only (hess == 1)")
+    if w_dev is None:
+        alpha = _era_alpha(era_weights, nes[:, 1:] - nes[:, :-1])
+    else:
+        alpha = _era_alpha_of(facts)
+    vals = grad.to(device=dev, dtype=torch.float32).contiguous()
     T = k_cuts if 0 < int(k_cuts) < nb - 1 else nb - 1
     # bins >= max_bins: the reference leaves those rows out of the histogram and sends them
     # right (frontier_cuda.cu:451, frontier_cpu.cpp:278-281, 464-470); here the subset's columns
-    # are copied with such bins set to max_bins, one extra plane bin that the scorer skips
+    # are copied with such bins set to max_bins, one extra plane bin that the scorer skips. Ids
+    # out of range are left to the gather kernel's own check (it raises "feature id").
     fid_gather, skip = fid, 0
-    sel = None
-    if K and N:
-        # ids out of range are left to the gather kernel's own check (it raises "feature id");
-        # index_select would read out of bounds with them
-        lo, hi = (int(v) for v in torch.aminmax(fid))
-        if 0 <= lo and hi < F:
-            sel = b_fm.index_select(0, fid.long())
-    if sel is not None and int(sel.max()) >= nb:
+    if facts["bin_over"] and not facts["bad_feature"]:
         if nb + 1 > 255:
             raise ValueError("bins >= max_bins need max_bins <= 254 on the HIP backend")
-        b_fm = torch.clamp(sel, max=nb).contiguous()
+        b_fm = torch.clamp(b_fm.index_select(0, fid.long()), max=nb).contiguous()
         F, ld_in = K, int(b_fm.stride(0))
         fid_gather, skip = torch.arange(K, dtype=torch.int32, device=dev), 1
-    del sel
     out_s = torch.full((M, K), float("-inf"), dtype=torch.float32, device=dev)
     out_t = torch.full((M, K), -1, dtype=torch.int32, device=dev)
     out_g = torch.zeros((M, K), dtype=torch.float32, device=dev)
@@ -144,37 +169,42 @@ def find_best_splits_batched_rowlist(bins, grad, hess, rows_index, node_row_spli
                    "pb_best_thresholds")
 
     _score_node_chunks(lib, b_fm, F, N, ld_in, fid_gather, fid, K, vals, rows, R, nrs, nes, M, E, nb + skip,
-                       T, p, _NODE_CHUNK, consume, "find_best_splits_batched_cuda")
+                       T, p, _NODE_CHUNK, consume, "find_best_splits_batched_cuda", rows_total=int(facts["rows"]))
     kernel_ms = (time.perf_counter() - t0) * 1e3
     return {"scores": out_s, "thresholds": out_t, "left_grad": out_g, "left_hess": out_h,
             "left_count": out_c, "kernel_ms": kernel_ms}
 
 
 def _score_node_chunks(lib, b_fm, F, N, ld_in, fid_gather, fid_score, K, vals, rows, R, nrs, nes, M, E, nb, T,
-                       p, chunk, consume, what, times=None):
+                       p, chunk, consume, what, times=None, rows_total=None):
     """For nodes [m0, m0 + chunk) at a time: pb_rowlist_gather of their listed rows (feature
     columns fid_gather of b_fm), pb_round_begin / pb_hist_build / pb_des_score over them (the
     candidates' feature ids are fid_score), then consume(m0, U, max_nodes, cand, cnt, gp) with
     the candidate records [max_nodes][K][T] and the histogram planes, before the chunk's
     context is released. Chunks whose lists hold no row are skipped. `times` (optional dict)
     accumulates the milliseconds of gather + histogram ("hist_ms") and of the scorer
-    ("score_ms"), from HIP events."""
+    ("score_ms"), from HIP events. `rows_total`: the listed rows of all nodes, where known."""
     dev = b_fm.device
     # rows listed per node (the gather places exactly these when the segments are consistent)
-    node_rows = (nes[:, E] - nes[:, 0]).to(torch.int64).clamp_min(0).cpu()
+    if rows_total is None or M > chunk:
+        node_rows = (nes[:, E] - nes[:, 0]).to(torch.int64).clamp_min(0).cpu()
     s = _hip.stream_ptr()
     for m0 in range(0, M, chunk):
         m1 = min(M, m0 + chunk)
         U = m1 - m0
-        cap = int(node_rows[m0:m1].sum())
+        cap = rows_total if rows_total is not None and M <= chunk else int(node_rows[m0:m1].sum())
         if cap == 0:
             continue
         ld = (cap + 15) // 16 * 16
-        b = torch.zeros((K, ld), dtype=torch.uint8, device=dev)
-        preds = torch.zeros(ld, dtype=torch.float32, device=dev)
-        nid = torch.full((ld,), -1, dtype=torch.int16, device=dev)  # 0xFFFF: rows in no node
-        era_off_dev = torch.empty(E + 1, dtype=torch.int32, device=dev)
-        work = torch.empty(int(lib.pb_rowlist_work_elems(U, E)), dtype=torch.int32, device=dev)
+        # the gather fills positions [0, cap); the padding rows hold bin 0, value 0 and no node (0xFFFF)
+        b = torch.empty((K, ld), dtype=torch.uint8, device=dev)
+        preds = torch.empty(ld, dtype=torch.float32, device=dev)
+        nid = torch.empty(ld, dtype=torch.int16, device=dev)
+        b[:, cap:], preds[cap:], nid[cap:] = 0, 0.0, -1
+        # era offsets, then the workspace whose first four words are the status: read back together
+        w0 = (E + 4) // 4 * 4
+        meta = torch.empty(w0 + int(lib.pb_rowlist_work_elems(U, E)), dtype=torch.int32, device=dev)
+        era_off_dev, work = meta[:E + 1], meta[w0:]
         ev = [torch.cuda.Event(enable_timing=True) for _ in range(3)] if times is not None else None
         if ev:
             ev[0].record()
@@ -182,8 +212,9 @@ def _score_node_chunks(lib, b_fm, F, N, ld_in, fid_gather, fid_score, K, vals, r
                                          rows.data_ptr(), R, nrs.data_ptr(), nes.data_ptr(), m0, m1, E,
                                          b.data_ptr(), ld, preds.data_ptr(), nid.data_ptr(),
                                          era_off_dev.data_ptr(), work.data_ptr(), s), "pb_rowlist_gather")
-        _check_status(work, what)
-        era_off = np.ascontiguousarray(era_off_dev.cpu().numpy())
+        meta_np = meta[:w0 + 4].cpu().numpy()
+        _check_status(meta_np[w0:], what)
+        era_off = np.ascontiguousarray(meta_np[:E + 1])
         Rc = int(era_off[E])
         if Rc == 0:
             continue

@@ -282,14 +282,6 @@ __device__ __forceinline__ void transpose4x4_bytes(const uint32_t (&r)[4], uint3
     c[3] = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
 }
 
-// 0x80 in every byte of x that is >= limit (1 <= limit <= 255)
-__device__ __forceinline__ uint32_t bytes_at_least(uint32_t x, uint32_t limit) {
-    const uint32_t low = x & 0x7f7f7f7fu;
-    const uint32_t hit = limit <= 128u ? ((low + (128u - limit) * 0x01010101u) | x)
-                                       : ((low + (256u - limit) * 0x01010101u) & x);
-    return hit & 0x80808080u;
-}
-
 __global__ __launch_bounds__(kBlock) void transpose_bins_kernel(const uint8_t* __restrict__ src, int64_t n,
                                                             int64_t stride, int32_t F,
                                                             const int64_t* __restrict__ perm,

@@ -972,9 +972,15 @@ int pb_frontier_set(pb_ctx* c, int32_t depth, int32_t num_active, const int32_t*
         return fail(PB_ERR_RANGE, "pb_frontier_set: num_active above the frontier bound of this depth");
     if (tree_size < 1 || tree_size > (1 << (c->d.max_depth + 1)))
         return fail(PB_ERR_RANGE, "pb_frontier_set: tree_size out of range");
+    if (!node_ids_host) {  // ids 0, 1, ..: set on the stream, nothing to wait for
+        if (num_active > tree_size) return fail(PB_ERR_RANGE, "pb_frontier_set: node id out of range");
+        PB_HIP(pb::launch_frontier_set(c->st, depth, num_active, tree_size, c->ids[depth & 1], (hipStream_t)stream),
+               "frontier_set launch");
+        return PB_OK;
+    }
     std::vector<int32_t> ids(std::max(num_active, 1));
     for (int i = 0; i < num_active; ++i) {
-        ids[i] = node_ids_host ? node_ids_host[i] : i;
+        ids[i] = node_ids_host[i];
         if (ids[i] < 0 || ids[i] >= tree_size) return fail(PB_ERR_RANGE, "pb_frontier_set: node id out of range");
     }
     hipStream_t s = (hipStream_t)stream;
@@ -1530,6 +1536,19 @@ int pb_rowlist_gather(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, con
                                      node_era_splits, node_begin, node_end, E, out_bins, out_ld,
                                      out_values, out_slot, era_off, work, (hipStream_t)stream),
            "rowlist gather launch");
+    return PB_OK;
+}
+
+int pb_rowlist_facts_get(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, const int32_t* feats, int32_t K,
+                         const float* hess, int64_t n_hess, const float* weights, const int32_t* node_era_splits,
+                         int32_t M, int32_t E, int32_t limit, pb_rowlist_facts* out, void* stream) {
+    if (N < 0 || ld < N || F < 0 || K < 0 || n_hess < 0 || M < 1 || E < 1 || limit < 1 || limit > 255)
+        return fail(PB_ERR_INVALID, "pb_rowlist_facts_get: bad shape");
+    if ((!bins && N > 0 && K > 0) || (!feats && K > 0) || (!hess && n_hess > 0) || !weights || !node_era_splits || !out)
+        return fail(PB_ERR_INVALID, "pb_rowlist_facts_get: null argument");
+    PB_HIP(pb::launch_rowlist_facts(bins, N, ld, F, feats, K, hess, n_hess, weights, node_era_splits, M, E, limit, out,
+                                    (hipStream_t)stream),
+           "rowlist facts launch");
     return PB_OK;
 }
 

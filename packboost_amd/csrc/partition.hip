@@ -309,6 +309,13 @@ __global__ __launch_bounds__(kBlock) void round_end_kernel(const uint16_t* __res
     }
 }
 
+__global__ __launch_bounds__(kBlock) void frontier_set_kernel(Frontier* st, int32_t depth, int32_t num_active,
+                                                          int32_t tree_size, int32_t* ids) {
+    for (int i = threadIdx.x; i < num_active; i += kBlock) ids[i] = i;
+    for (int d = depth + (int)threadIdx.x; d <= PB_MAX_DEPTH; d += kBlock) st->u_active[d] = d == depth ? num_active : 0;
+    if (threadIdx.x == 0) st->tree_size = tree_size;
+}
+
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 int grid_for(int64_t work, int per_block, int cap) {
@@ -344,6 +351,12 @@ hipError_t launch_partition_end(const uint8_t* bins, int64_t ld, int32_t nibble,
 hipError_t launch_select_subsets(const pb_round_header* prev, int32_t D, int32_t K,
                                  const int32_t* window, int32_t* feats, hipStream_t s) {
     hipLaunchKernelGGL(select_subsets_kernel, dim3(1), dim3(kBlock), 0, s, prev, D, K, window, feats);
+    return hipGetLastError();
+}
+
+hipError_t launch_frontier_set(Frontier* st, int32_t depth, int32_t num_active, int32_t tree_size, int32_t* ids,
+                               hipStream_t s) {
+    hipLaunchKernelGGL(frontier_set_kernel, dim3(1), dim3(kBlock), 0, s, st, depth, num_active, tree_size, ids);
     return hipGetLastError();
 }
 

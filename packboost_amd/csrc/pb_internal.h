@@ -113,6 +113,14 @@ __device__ __forceinline__ float exact_recip(float n) {
     return __builtin_fmaf(e, r, r);
 }
 
+// 0x80 in every byte of x that is >= limit (1 <= limit <= 255)
+__device__ __forceinline__ uint32_t bytes_at_least(uint32_t x, uint32_t limit) {
+    const uint32_t low = x & 0x7f7f7f7fu;
+    const uint32_t hit = limit <= 128u ? ((low + (128u - limit) * 0x01010101u) | x)
+                                       : ((low + (256u - limit) * 0x01010101u) & x);
+    return hit & 0x80808080u;
+}
+
 // Per active node of the current depth, read by the partition kernel.
 struct SplitRule {
     int32_t feature;    // -1: node did not split
@@ -412,6 +420,12 @@ hipError_t launch_rowlist_gather(const uint8_t* bins, int64_t N, int64_t ld, int
                                  const int32_t* nes, int32_t m0, int32_t m1, int32_t E,
                                  uint8_t* out_bins, int64_t out_ld, float* out_values,
                                  uint16_t* out_slot, int32_t* era_off, int32_t* work, hipStream_t s);
+hipError_t launch_rowlist_facts(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, const int32_t* feats, int32_t K,
+                                const float* hess, int64_t n_hess, const float* weights, const int32_t* nes, int32_t M,
+                                int32_t E, int32_t limit, pb_rowlist_facts* out, hipStream_t s);
+// num_active node ids 0, 1, .. as the frontier of a depth (pb_frontier_set without ids).
+hipError_t launch_frontier_set(Frontier* st, int32_t depth, int32_t num_active, int32_t tree_size, int32_t* ids,
+                               hipStream_t s);
 hipError_t launch_best_thresholds(const pb_candidate* cand, int32_t M, int32_t K, int32_t T,
                                   float* score, int32_t* thr, float* left_grad, float* left_hess,
                                   int64_t* left_count, hipStream_t s);

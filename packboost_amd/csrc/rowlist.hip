@@ -297,22 +297,40 @@ __global__ void rl_sizes_kernel(const int32_t* nrs, const int32_t* nes, int64_t 
     }
 }
 
-// One wavefront per segment: its rows to their era-major positions with K bins each.
+// One wavefront per (segment, block of kGatherFeats features): the segment's rows to their era-major
+// positions, with those features' bins (the first block also moves values and slots). The block's
+// loads of a row are in flight together; a wavefront per segment left 800 segments of 250 rows and
+// 100 features to 3 waves a CU, each waiting on one byte load after another: 416 us for those, 50 us so.
+constexpr int kGatherFeats = 8;
+
 __global__ __launch_bounds__(kRlBlock) void rl_gather_kernel(
-    const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F, const int32_t* feats, int32_t K,
+    const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F, const int32_t* __restrict__ feats, int32_t K,
     const float* __restrict__ values, const int32_t* __restrict__ rows, int64_t R, const int32_t* nrs,
-    const int32_t* nes, int32_t m0, int32_t m1, int32_t E, const int32_t* scan, uint8_t* out_bins,
-    int64_t out_ld, float* out_values, uint16_t* out_slot, int32_t* status) {
+    const int32_t* nes, int32_t m0, int32_t m1, int32_t E, const int32_t* scan, uint8_t* __restrict__ out_bins,
+    int64_t out_ld, float* __restrict__ out_values, uint16_t* __restrict__ out_slot, int32_t* status) {
     const int lane = threadIdx.x & (kWave - 1);
     const int32_t Mc = m1 - m0;
-    const int64_t n = (int64_t)Mc * E;
+    const int64_t blocks = (K + kGatherFeats - 1) / kGatherFeats > 0 ? (K + kGatherFeats - 1) / kGatherFeats : 1;
+    const int64_t n = (int64_t)Mc * E * blocks;
     bool bad_row = false, bad_feat = false, over = false;
-    for (int64_t j = (int64_t)blockIdx.x * kRlWaves + threadIdx.x / kWave; j < n;
-         j += (int64_t)gridDim.x * kRlWaves) {
+    for (int64_t x = (int64_t)blockIdx.x * kRlWaves + threadIdx.x / kWave; x < n;
+         x += (int64_t)gridDim.x * kRlWaves) {
+        // an era's segments are next to one another for one feature block: its column lines are shared
+        const int64_t fb = x / ((int64_t)Mc * E), j = x - fb * ((int64_t)Mc * E);
         const int32_t e = (int32_t)(j / Mc), sl = (int32_t)(j - (int64_t)e * Mc);
+        const int k0 = (int)fb * kGatherFeats;
         int64_t lo, hi;
         seg_range(nrs, nes, E, R, m0 + sl, e, lo, hi);
         const int64_t dst = scan[2 * j];
+        const uint8_t* col[kGatherFeats];
+        bool ok[kGatherFeats];
+#pragma unroll
+        for (int q = 0; q < kGatherFeats; ++q) {
+            const int32_t f = k0 + q < K ? feats[k0 + q] : 0;
+            ok[q] = k0 + q < K && f >= 0 && f < F;
+            bad_feat |= k0 + q < K && !ok[q] && hi > lo;
+            col[q] = bins + (ok[q] ? (int64_t)f * ld : 0);
+        }
         for (int64_t i = lo + lane; i < hi; i += kWave) {
             const int64_t d = dst + (i - lo);
             if (d < 0 || d >= out_ld) {
@@ -322,14 +340,16 @@ __global__ __launch_bounds__(kRlBlock) void rl_gather_kernel(
             const int32_t r = rows[i];
             const bool rok = r >= 0 && r < N;
             bad_row |= !rok;
-            out_values[d] = values[i];
-            out_slot[d] = (uint16_t)sl;
-            for (int k = 0; k < K; ++k) {
-                const int32_t f = feats[k];
-                const bool fok = f >= 0 && f < F;
-                bad_feat |= !fok;
-                out_bins[(int64_t)k * out_ld + d] = (rok && fok) ? bins[(int64_t)f * ld + r] : (uint8_t)0;
+            if (fb == 0) {
+                out_values[d] = values[i];
+                out_slot[d] = (uint16_t)sl;
             }
+            uint8_t b[kGatherFeats];
+#pragma unroll
+            for (int q = 0; q < kGatherFeats; ++q) b[q] = rok && ok[q] ? col[q][r] : (uint8_t)0;
+#pragma unroll
+            for (int q = 0; q < kGatherFeats; ++q)
+                if (k0 + q < K) out_bins[(int64_t)(k0 + q) * out_ld + d] = b[q];
         }
     }
     if (bad_row) raise_status(status, kBadRow);
@@ -345,26 +365,41 @@ __global__ void rl_era_off_kernel(const int32_t* scan, int32_t Mc, int32_t E, in
 
 // Per (node, feature): frontier_cuda.cu:537-560's pick over the thresholds in their order
 // (score within 1e-12 of the best: the larger left count, then the larger threshold wins; a
-// non-finite best leaves threshold -1 and zero sums).
-__global__ void rl_best_kernel(const pb_candidate* cand, int64_t MK, int32_t T, float* score, int32_t* thr,
-                               float* left_grad, float* left_hess, int64_t* left_count) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= MK) return;
+// non-finite best leaves threshold -1 and zero sums). One wavefront each: 64 candidate records are
+// loaded together and the pick runs over them in order on values every lane reads from the lane
+// that holds them (the rule is not transitive, so the order is kept); a lane walking its own
+// 127 records of 32 bytes waited on each (72 us for 16 x 100, 16 us so).
+__global__ __launch_bounds__(kRlBlock) void rl_best_kernel(const pb_candidate* __restrict__ cand, int64_t MK, int32_t T,
+                                                        float* __restrict__ score, int32_t* __restrict__ thr,
+                                                        float* __restrict__ left_grad, float* __restrict__ left_hess,
+                                                        int64_t* __restrict__ left_count) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t i = (int64_t)blockIdx.x * kRlWaves + threadIdx.x / kWave;
+    if (i >= MK) return;  // whole wavefronts
     float bs = -__builtin_inff(), blg = 0.0f;
-    int32_t bt = -1;
-    int64_t bl = 0;
-    for (int t = 0; t < T; ++t) {
-        const pb_candidate c = cand[i * T + t];
-        if (!c.valid) continue;
-        const float sc = c.score;
-        const int64_t lc = c.left_total;
-        bool better = sc > bs;
-        if (!better && fabsf(sc - bs) <= 1e-12f) better = lc > bl || (lc == bl && c.threshold > bt);
-        if (better) {
-            bs = sc;
-            bt = c.threshold;
-            blg = c.left_grad;
-            bl = lc;
+    int32_t bt = -1, bl = 0;
+    for (int t0 = 0; t0 < T; t0 += kWave) {
+        pb_candidate c;
+        c.valid = 0;
+        c.score = c.left_grad = 0.0f;
+        c.threshold = -1;
+        c.left_total = 0;
+        if (t0 + lane < T) c = cand[i * T + t0 + lane];
+        uint64_t todo = __ballot(c.valid != 0);
+        while (todo) {
+            const int l = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const float sc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.score), l));
+            const int32_t lc = __builtin_amdgcn_readlane(c.left_total, l);
+            const int32_t th = __builtin_amdgcn_readlane(c.threshold, l);
+            bool better = sc > bs;
+            if (!better && fabsf(sc - bs) <= 1e-12f) better = lc > bl || (lc == bl && th > bt);
+            if (better) {
+                bs = sc;
+                bt = th;
+                blg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.left_grad), l));
+                bl = lc;
+            }
         }
     }
     if (!(bs == bs) || isinf(bs)) {
@@ -372,11 +407,100 @@ __global__ void rl_best_kernel(const pb_candidate* cand, int64_t MK, int32_t T, 
         blg = 0.0f;
         bl = 0;
     }
+    if (lane) return;
     score[i] = bs;
     thr[i] = bt;
     left_grad[i] = blg;
-    left_hess[i] = (float)bl;  // squared loss: hess == 1 per row
+    left_hess[i] = (float)(int64_t)bl;  // squared loss: hess == 1 per row
     left_count[i] = bl;
+}
+
+// What a call's inputs must satisfy, looked up in one launch (RowlistFacts, cleared by the caller):
+// workgroup 0 covers the weights and row counts, the others hess and the drawn columns' bins.
+__global__ __launch_bounds__(kRlBlock) void rl_facts_kernel(
+    const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F, const int32_t* __restrict__ feats, int32_t K,
+    const float* __restrict__ hess, int64_t n_hess, const float* __restrict__ weights, const int32_t* __restrict__ nes,
+    int32_t M, int32_t E, uint32_t limit, pb_rowlist_facts* out) {
+    const int lane = threadIdx.x & (kWave - 1);
+    if (blockIdx.x == 0) {
+        __shared__ double s_lo[kRlWaves], s_hi[kRlWaves];
+        __shared__ unsigned long long s_rows[kRlWaves];
+        double lo = __builtin_inf(), hi = -__builtin_inf();
+        unsigned long long total = 0ull;
+        bool stray = false, counted = false, unit = true;
+        for (int64_t x = threadIdx.x; x < (int64_t)M * E; x += kRlBlock) {
+            const int64_t s = x / E, e = x - s * E;
+            const int32_t c = nes[s * (E + 1) + e + 1] - nes[s * (E + 1) + e];
+            const float w = weights[x];
+            if (c > 0) {
+                const double d = (double)w - (double)c;
+                counted = true;
+                unit &= w == 1.0f;
+                lo = fmin(lo, d);
+                hi = fmax(hi, d);
+                if (isnan(w)) lo = -__builtin_inf(), hi = __builtin_inf();  // no common era_alpha
+            } else {
+                stray |= !(w == 0.0f);
+            }
+            if (e == 0) {
+                const int64_t rows = (int64_t)nes[s * (E + 1) + E] - nes[s * (E + 1)];
+                total += rows > 0 ? (unsigned long long)rows : 0ull;
+            }
+        }
+        for (int32_t k = threadIdx.x; k < K; k += kRlBlock)
+            if (feats[k] < 0 || feats[k] >= F) out->bad_feature = 1;
+        if (stray) out->stray_weight = 1;
+        if (counted) out->counted = 1;
+        if (!unit) out->not_unit = 1;
+#pragma unroll
+        for (int m = 1; m < kWave; m <<= 1) {
+            lo = fmin(lo, __shfl_xor(lo, m));
+            hi = fmax(hi, __shfl_xor(hi, m));
+            total += __shfl_xor(total, m);
+        }
+        if (lane == 0) {
+            s_lo[threadIdx.x / kWave] = lo;
+            s_hi[threadIdx.x / kWave] = hi;
+            s_rows[threadIdx.x / kWave] = total;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < kRlWaves; ++w) {
+                lo = fmin(lo, s_lo[w]);
+                hi = fmax(hi, s_hi[w]);
+                total += s_rows[w];
+            }
+            out->alpha_lo = lo;
+            out->alpha_hi = hi;
+            out->rows = (int64_t)total;
+        }
+        return;
+    }
+    const int64_t t = (int64_t)(blockIdx.x - 1) * kRlBlock + threadIdx.x;
+    const int64_t stride = (int64_t)(gridDim.x - 1) * kRlBlock;
+    bool bad = false;
+    for (int64_t i = t; i < n_hess; i += stride) bad |= !(hess[i] == 1.0f);
+    if (bad) out->bad_hess = 1;
+    // 16 bytes of a drawn column at a time (byte by byte at its end): any alignment
+    struct __attribute__((packed)) Bytes16 {
+        uint32_t w[4];
+    };
+    const int64_t per_col = (N + 15) / 16;
+    bool over = false;
+    for (int64_t x = t; x < per_col * K; x += stride) {
+        const int64_t k = x / per_col, r = (x - k * per_col) * 16;
+        const int32_t f = feats[k];
+        if (f < 0 || f >= F) continue;
+        const uint8_t* p = bins + (int64_t)f * ld + r;
+        if (r + 16 <= N) {
+            const Bytes16 v = *reinterpret_cast<const Bytes16*>(p);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) over |= bytes_at_least(v.w[q], limit) != 0u;
+        } else {
+            for (int64_t b = r; b < N; ++b) over |= p[b - r] >= limit;
+        }
+    }
+    if (over) out->bin_over = 1;
 }
 
 int grid_of(int64_t work, int64_t per_block, int64_t cap) {
@@ -476,7 +600,8 @@ hipError_t launch_rowlist_gather(const uint8_t* bins, int64_t N, int64_t ld, int
     hipLaunchKernelGGL(rl_sizes_kernel, dim3(grid_of(n, 256, 1 << 14)), dim3(256), 0, s, nrs, nes, R, m0, m1,
                        E, vals, status);
     scan_pairs(vals, n, tiles, scan, s);
-    hipLaunchKernelGGL(rl_gather_kernel, dim3(grid_of(n, kRlWaves, 1 << 16)), dim3(kRlBlock), 0, s, bins, N,
+    const int64_t units = n * std::max<int64_t>(1, (K + kGatherFeats - 1) / kGatherFeats);
+    hipLaunchKernelGGL(rl_gather_kernel, dim3(grid_of(units, kRlWaves, 1 << 16)), dim3(kRlBlock), 0, s, bins, N,
                        ld, F, feats, K, values, rows, R, nrs, nes, m0, m1, E, scan, out_bins, out_ld,
                        out_values, out_slot, status);
     hipLaunchKernelGGL(rl_era_off_kernel, dim3(grid_of((int64_t)E + 1, 256, 1 << 14)), dim3(256), 0, s, scan,
@@ -488,8 +613,18 @@ hipError_t launch_best_thresholds(const pb_candidate* cand, int32_t M, int32_t K
                                   float* score, int32_t* thr, float* left_grad, float* left_hess,
                                   int64_t* left_count, hipStream_t s) {
     const int64_t n = (int64_t)M * K;
-    hipLaunchKernelGGL(rl_best_kernel, dim3(grid_of(n, 256, 1 << 24)), dim3(256), 0, s, cand, n, T, score,
-                       thr, left_grad, left_hess, left_count);
+    if ((n + kRlWaves - 1) / kRlWaves > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(rl_best_kernel, dim3((unsigned)((n + kRlWaves - 1) / kRlWaves)), dim3(kRlBlock), 0, s, cand, n,
+                       T, score, thr, left_grad, left_hess, left_count);
+    return hipGetLastError();
+}
+
+hipError_t launch_rowlist_facts(const uint8_t* bins, int64_t N, int64_t ld, int32_t F, const int32_t* feats, int32_t K,
+                                const float* hess, int64_t n_hess, const float* weights, const int32_t* nes, int32_t M,
+                                int32_t E, int32_t limit, pb_rowlist_facts* out, hipStream_t s) {
+    const int64_t work = std::max<int64_t>(n_hess, (N + 15) / 16 * K);
+    hipLaunchKernelGGL(rl_facts_kernel, dim3(1 + grid_of(work, kRlBlock, 2048)), dim3(kRlBlock), 0, s, bins, N, ld, F,
+                       feats, K, hess, n_hess, weights, nes, M, E, (uint32_t)limit, out);
     return hipGetLastError();
 }
 

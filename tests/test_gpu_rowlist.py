@@ -321,3 +321,92 @@ def test_best_thresholds_tie_break(hip):
     assert got_t[0, 0] == -1 and np.isneginf(got_s[0, 0])
     assert got_t[1, 0] == -1 and np.isposinf(got_s[1, 0]) and got_c[1, 0] == 0
     assert got_t[1, 2] == -1
+
+
+@pytest.mark.parametrize("nb,T", [(5, 4), (64, 63), (65, 64), (129, 128), (200, 199)])
+def test_best_thresholds_order(hip, nb, T):
+    """The per-(node, feature) pick over thresholds that tie, nearly tie (within 1e-12, where the
+    scan's order decides), are invalid or infinite, at every record window edge, against the scan
+    in Python: exact."""
+    import torch
+
+    rng = np.random.default_rng(nb)
+    M, K = 3, 7
+    rec = np.zeros((M, K, T), dtype=hip.CANDIDATE_DTYPE)
+    rec["score"] = rng.integers(0, 4, (M, K, T)).astype(np.float32) * np.float32(4e-13)
+    rec["score"][1] = rng.integers(0, 3, (K, T)).astype(np.float32)
+    rec["score"][2, 0, :] = -np.inf
+    rec["score"][2, 1, T // 2] = np.inf
+    rec["score"][2, 2, 0] = np.nan
+    rec["left_total"] = rng.integers(0, 3, (M, K, T))
+    rec["left_grad"] = rng.standard_normal((M, K, T)).astype(np.float32)
+    rec["threshold"] = rng.permutation(T)[None, None, :]
+    rec["valid"] = rng.random((M, K, T)) < 0.8
+    rec["valid"][0, 0] = 0
+    cand = torch.from_numpy(rec.view(np.uint8).reshape(-1)).cuda()
+    s, g, h = (torch.empty((M, K), dtype=torch.float32, device="cuda") for _ in range(3))
+    t = torch.empty((M, K), dtype=torch.int32, device="cuda")
+    c = torch.empty((M, K), dtype=torch.int64, device="cuda")
+    hip.check(hip.load().pb_best_thresholds(cand.data_ptr(), M, K, T, s.data_ptr(), t.data_ptr(), g.data_ptr(),
+                                            h.data_ptr(), c.data_ptr(), hip.stream_ptr()), "pb_best_thresholds")
+    for m in range(M):
+        for k in range(K):
+            bs, bt, bg, bl = np.float32(-np.inf), -1, np.float32(0), 0
+            for r in rec[m, k]:
+                if not r["valid"]:
+                    continue
+                sc, lc, th = r["score"], int(r["left_total"]), int(r["threshold"])
+                with np.errstate(invalid="ignore"):
+                    near = abs(np.float32(sc - bs)) <= np.float32(1e-12)
+                if sc > bs or (near and (lc > bl or (lc == bl and th > bt))):
+                    bs, bt, bg, bl = sc, th, r["left_grad"], lc
+            if not np.isfinite(bs):
+                bt, bg, bl = -1, np.float32(0), 0
+            got = (s[m, k].item(), t[m, k].item(), g[m, k].item(), h[m, k].item(), c[m, k].item())
+            assert got == (float(bs), bt, float(bg), float(bl), bl), (m, k, got)
+
+
+@pytest.mark.parametrize("what", ["hess", "stray", "alpha", "nan", "feature", "segment", "float64"])
+def test_split_finder_input_checks(hip, what):
+    """Inputs the row-list split finder refuses (and float64 weights, which it takes)."""
+    import torch
+
+    from packboost_amd import backends
+
+    p = make_problem(11, 900, 9, 4, 5, 3)
+    ner = node_era_rows(p)
+    ner[1][2] = ner[1][2][:0]  # an era without rows
+    rows, nrs, nes = _rowlist_inputs(p, ner)
+    dev = torch.device("cuda")
+    bins = torch.from_numpy(np.ascontiguousarray(p["bins"].T)).to(dev)
+    g = torch.from_numpy(p["grad"]).to(dev)[rows.long()]
+    hess = torch.ones_like(g)
+    cnt = (nes[:, 1:] - nes[:, :-1]).float()
+    w = torch.where(cnt > 0, cnt + 2.5, torch.zeros_like(cnt))
+    ids = torch.arange(9, dtype=torch.int32, device=dev)
+    want = None
+    if what == "hess":
+        hess[7], want = 0.5, "squared loss"
+    elif what == "stray":
+        w[1, 2], want = 1.0, "without rows"
+    elif what in ("alpha", "nan"):
+        w[0, 0], want = (w[0, 0] + 1 if what == "alpha" else float("nan")), "one era_alpha"
+    elif what == "feature":
+        ids[3], want = 9, "feature id"
+    elif what == "segment":
+        nes[0, 1], want = nes[0, 4] + 10_000, "segment"
+        w = (nes[:, 1:] > nes[:, :-1]).float()
+    else:
+        w = w.double()
+
+    def call():
+        z = torch.zeros(3, device=dev)
+        return backends.find_best_splits_batched_cuda(bins, g, hess, rows, nrs, nes, w, z, z, z.long(), ids, 5, 0,
+                                                      "mass", 1e-3, 0.4, 0.1, 5)
+    if want is None:
+        got, w = call(), w.float()
+        ref = call()
+        assert all(torch.equal(got[k], ref[k]) for k in ("scores", "thresholds", "left_grad", "left_count"))
+    else:
+        with pytest.raises(RuntimeError, match=want):
+            call()
