@@ -458,7 +458,8 @@ int64_t pb_rowlist_work_elems(int32_t num_nodes, int32_t num_eras);
  * bin[feat[s]][row] <= thr[s] (left) and the rest (right), in list order. left_index and
  * right_index receive the node-major, era-minor concatenation (capacity entries each; R
  * suffices for disjoint segments); left_splits / right_splits int32 [S][E+1] are absolute
- * offsets into them (entry [S-1][E] = the total). */
+ * offsets into them (entry [S-1][E] = the total). work_dev[4..5] are left with the left and right
+ * totals. */
 int pb_rowlist_partition(const uint8_t* bins_dev, int64_t N, int64_t ld, int32_t F,
                          const int32_t* rows_dev, int64_t R, const int32_t* node_row_splits_dev,
                          const int32_t* node_era_splits_dev, int32_t S, int32_t E,

@@ -289,8 +289,9 @@ def partition_frontier_rowlist(bins, rows_index, node_row_splits, node_era_split
                                         nes.data_ptr(), S, E, feat.data_ptr(), thr.data_ptr(),
                                         left.data_ptr(), right.data_ptr(), R, ls.data_ptr(), rs.data_ptr(),
                                         work.data_ptr(), _hip.stream_ptr()), "pb_rowlist_partition")
-    _check_status(work, "partition_frontier_cuda")
-    nl, nr = int(ls[-1, -1]), int(rs[-1, -1])
+    head = work[:6].cpu().numpy()  # status words, then the left and right row totals
+    _check_status(head[:4], "partition_frontier_cuda")
+    nl, nr = int(head[4]), int(head[5])
     return {"left_index": left[:nl], "right_index": right[:nr], "left_splits": ls, "right_splits": rs}
 
 

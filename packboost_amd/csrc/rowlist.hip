@@ -227,9 +227,11 @@ __global__ __launch_bounds__(kRlBlock) void rl_tile_scan_kernel(const int32_t* v
     }
 }
 
-// [S][E+1] split offsets from the scan (node s's entries are scan pairs s*E .. s*E + E).
+// [S][E+1] split offsets from the scan (node s's entries are scan pairs s*E .. s*E + E); totals [2]:
+// the left and right rows of all segments.
 __global__ void rl_splits_kernel(const int32_t* scan, int32_t S, int32_t E, int32_t* left_splits,
-                                 int32_t* right_splits) {
+                                 int32_t* right_splits, int32_t* totals) {
+    if (blockIdx.x == 0 && threadIdx.x < 2) totals[threadIdx.x] = scan[2 * (int64_t)S * E + threadIdx.x];
     const int64_t n = (int64_t)S * (E + 1);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t s = i / (E + 1), e = i - s * (E + 1);
@@ -542,7 +544,7 @@ void rowlist_partition_stages(const uint8_t* bins, int64_t N, int64_t ld, int32_
                        S, E, feat, thr, vals, status);
     scan_pairs(vals, n, tiles, scan, s);
     hipLaunchKernelGGL(rl_splits_kernel, dim3(grid_of((int64_t)S * (E + 1), 256, 1 << 14)), dim3(256), 0, s,
-                       scan, S, E, left_splits, right_splits);
+                       scan, S, E, left_splits, right_splits, vals);  // the scan is done with the counts
     hipLaunchKernelGGL(rl_scatter_kernel, dim3(g), dim3(kRlBlock), 0, s, bins, N, ld, F, rows, R, nrs, nes,
                        S, E, feat, thr, scan, left_out, right_out, cap, status);
 }

@@ -410,3 +410,36 @@ def test_split_finder_input_checks(hip, what):
     else:
         with pytest.raises(RuntimeError, match=want):
             call()
+
+
+@pytest.mark.parametrize("sizes", [[0], [1], [63, 64, 65], [255, 0, 256, 257], [1000, 3, 511, 512, 513]], ids=str)
+def test_partition_totals(hip, sizes):
+    """Segments of 0 to 1000 rows at wavefront edges, and a row id and a feature that are refused:
+    the lists equal NumPy's stable split, their lengths the totals read back with the status."""
+    import torch
+
+    from packboost_amd import backends
+
+    dev = torch.device("cuda")
+    rng = np.random.default_rng(sum(sizes))
+    N, F, E, S = 3000, 5, len(sizes), 2
+    bins = rng.integers(0, 9, (F, N), dtype=np.uint8)
+    ner = [[rng.integers(0, N, n) for n in sizes] for _ in range(S)]
+    rows, nrs, nes = _rowlist_inputs(None, ner)
+    feat, thr = np.array([4, 1], np.int32), np.array([3, -1], np.int32)
+    call = lambda r, f: backends.partition_frontier_cuda(  # noqa: E731
+        torch.from_numpy(bins).to(dev), r, nrs, nes, torch.from_numpy(f).to(dev), torch.from_numpy(thr).to(dev))
+    out = call(rows, feat)
+    go = [[bins[feat[s], r] <= thr[s] for r in ner[s]] for s in range(S)]
+    for key, pick in (("left", lambda g: g), ("right", lambda g: ~g)):
+        lists = [r[pick(g)] for s in range(S) for r, g in zip(ner[s], go[s])]
+        np.testing.assert_array_equal(out[f"{key}_index"].cpu().numpy(), np.concatenate(lists))
+        ends = np.concatenate([[0], np.cumsum([len(x) for x in lists])])
+        np.testing.assert_array_equal(out[f"{key}_splits"].cpu().numpy(), [ends[s * E:s * E + E + 1] for s in range(S)])
+    if sum(sizes):
+        bad = rows.clone()
+        bad[-1] = N
+        with pytest.raises(RuntimeError, match="row id"):
+            call(bad, feat)
+        with pytest.raises(RuntimeError, match="feature id"):
+            call(rows, np.array([4, F], np.int32))
