@@ -34,6 +34,8 @@ struct pb_ctx {
     int32_t S;
     int32_t* seg_info_dev;  // [S][4] per work segment: first row, end row, era, slot of a
                             // split era (-1: the era is one segment)
+    int32_t S_fine;         // finer segments of the same eras for narrow frontiers (0: none)
+    int32_t* seg_fine_dev;  // [S_fine][4]
     float* win_sum;         // |grad| sum per window of pb::kGradWinRows rows (round_begin)
     int32_t* sh_era;        // [E] fixed-point gradient scale exponent of each era
     int32_t n_acc;          // eras split into several segments
@@ -155,6 +157,7 @@ void free_ctx(pb_ctx* c) {
     (void)hipFree(c->ss.cnt_r);
     (void)hipFree(c->ss.base);
     (void)hipFree(c->seg_info_dev);
+    (void)hipFree(c->seg_fine_dev);
     (void)hipFree(c->acc_era_dev);
     (void)hipFree(c->acc_cnt);
     (void)hipFree(c->acc_g);
@@ -261,10 +264,27 @@ int pb_ctx_create(const pb_dims* dims, const int32_t* era_off_host, pb_ctx** out
     c->S = (int32_t)(seg_info.size() / 4);
     c->n_acc = (int32_t)acc_era.size();
     c->cnt32 = max_era > pb::kMaxEraRowsDirect;
+    // finer parts of about 1/64 of the rows for narrow frontiers, when every era is split (hist_build)
+    std::vector<int32_t> seg_fine;
+    if (c->n_acc == d.num_eras) {
+        const int64_t rows = std::max<int64_t>(1024, (d.num_rows + 63) / 64);
+        if (rows * 2 <= seg_rows)
+            for (int e = 0; e < d.num_eras; ++e) {
+                const int64_t len = era_off_host[e + 1] - era_off_host[e], parts = (len + rows - 1) / rows;
+                for (int64_t j = 0; j < parts; ++j) {
+                    seg_fine.push_back((int32_t)(era_off_host[e] + len * j / parts));
+                    seg_fine.push_back((int32_t)(era_off_host[e] + len * (j + 1) / parts));
+                    seg_fine.push_back(e);
+                    seg_fine.push_back(e);  // every era is split: slot e
+                }
+            }
+    }
+    c->S_fine = (int32_t)(seg_fine.size() / 4);
     const size_t acc_cells = (size_t)c->n_acc * c->umax * d.max_feats * d.max_bins;
 
     int rc = PB_OK;
-    if ((rc = dev_alloc(&c->seg_info_dev, std::max<size_t>(4, seg_info.size()), "alloc segments")) ||
+    if ((rc = dev_alloc(&c->seg_fine_dev, std::max<size_t>(4, seg_fine.size()), "alloc segments")) ||
+        (rc = dev_alloc(&c->seg_info_dev, std::max<size_t>(4, seg_info.size()), "alloc segments")) ||
         (rc = dev_alloc(&c->acc_era_dev, std::max<size_t>(1, acc_era.size()), "alloc segment slots")) ||
         (rc = dev_alloc(&c->acc_cnt, std::max<size_t>(1, acc_cells), "alloc segment sums")) ||
         (rc = dev_alloc(&c->acc_g, std::max<size_t>(1, acc_cells), "alloc segment sums"))) {
@@ -276,6 +296,8 @@ int pb_ctx_create(const pb_dims* dims, const int32_t* era_off_host, pb_ctx** out
         if (!seg_info.empty())
             e1 = hipMemcpy(c->seg_info_dev, seg_info.data(), sizeof(int32_t) * seg_info.size(),
                            hipMemcpyHostToDevice);
+        if (e1 == hipSuccess && !seg_fine.empty())
+            e1 = hipMemcpy(c->seg_fine_dev, seg_fine.data(), sizeof(int32_t) * seg_fine.size(), hipMemcpyHostToDevice);
         if (e1 == hipSuccess && !acc_era.empty())
             e1 = hipMemcpy(c->acc_era_dev, acc_era.data(), sizeof(int32_t) * acc_era.size(),
                            hipMemcpyHostToDevice);
@@ -416,6 +438,20 @@ int hist_build(pb_ctx* c, const uint8_t* bins, int64_t ld_bytes, int32_t nibble,
     int64_t need = 1;
     while (need < groups_k) need *= 2;  // no more groups than the features present need
     groups = std::min<int64_t>(groups, need);
+    // Enough workgroups to cover the chip: narrower tiles while a narrow frontier leaves fewer than
+    // 1024 items (200k rows x 100 features x 128 bins in 50 eras, depths 0-1: 4-feature tiles 19.6 /
+    // 20.1 us against 26.6 / 22.4 for the widest that fit), a wider one fewer than one per CU (10k
+    // rows x 20 features, depth 3: 8.4 against 10.3; at 416 items of 16 nodes a further halving lost,
+    // 25.4 against 22.6 us: every tile re-reads the rows' state). Up to two nodes, where a part's flush is
+    // short, eras that are all split go in finer parts too (one era of 200k rows x 64 features,
+    // depths 0-1: 16.3 / 17.3 us against 41.7 / 40.7 in 13 parts; twice as many parts 18.5 / 21.4,
+    // and from four nodes on the parts' global sums cost more than they save).
+    const int64_t want = max_nodes <= 4 ? 1024 : 256;
+    auto items = [&](int64_t segs, int64_t g) { return segs * node_tiles * ((K + g * P - 1) / (g * P)); };
+    const bool fine = c->S_fine > 0 && max_nodes <= 2 && items(c->S, groups) < want;
+    const int32_t S = fine ? c->S_fine : c->S;
+    if (c->force_ftile <= 0)
+        while (groups > 1 && items(S, groups) < want) groups /= 2;
     int clog2 = 0;
     if (c->force_copies > 0) {
         while ((1 << (clog2 + 1)) <= c->force_copies && clog2 < 5) ++clog2;
@@ -463,8 +499,8 @@ int hist_build(pb_ctx* c, const uint8_t* bins, int64_t ld_bytes, int32_t nibble,
         a.out_g = hist_grad;
         a.out_tot_g = hist_grad + to;
     }
-    a.seg_info = reinterpret_cast<const int4*>(c->seg_info_dev);
-    a.S = c->S;
+    a.seg_info = reinterpret_cast<const int4*>(fine ? c->seg_fine_dev : c->seg_info_dev);
+    a.S = S;
     a.acc_cnt = c->acc_cnt;
     a.acc_g = c->acc_g;
     a.acc_U = c->umax;  // active nodes < umax whatever max_nodes the caller passes

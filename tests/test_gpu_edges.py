@@ -300,3 +300,25 @@ def test_split_era_bins(hip, monkeypatch, nb):
             g.close()
     np.testing.assert_array_equal(planes[0][0], planes[1][0])
     np.testing.assert_array_equal(planes[0][1], planes[1][1])
+
+
+@pytest.mark.parametrize("N,K,nb,U", [(40_001, 7, 63, 1), (40_001, 7, 63, 2), (40_001, 40, 63, 3), (33_000, 3, 5, 2),
+                                      (70_003, 33, 128, 1), (20_000, 2, 9, 1)])
+def test_narrow_frontier_parts(hip, oracle_mod, N, K, nb, U):
+    """One era in finer parts and narrower feature tiles at one and two nodes (and a wider frontier,
+    which keeps the segments): the planes equal the oracle's, and a rebuild the first build's."""
+    p = make_problem(N + K, N, K, 1, nb, U, ragged=False)
+    p["era_off"], p["era"] = np.array([0, N], np.int32), np.zeros(N, np.int64)
+    feats = np.random.default_rng(K).permutation(K).astype(np.int32)
+    ref = oracle_mod.split_batch(p["bins"], p["grad"], node_era_rows(p), feats, nb, want_planes=True)
+    for layout in ("u8", "nibble") if nb <= 16 else ("u8",):
+        g = GpuDepth(hip, p, K, msl=1, layout=layout)
+        try:
+            for _ in range(2):
+                g.hist(feats)
+                cnt, gp = g.planes()
+                np.testing.assert_array_equal(cnt, ref.planes[0])
+                err = np.abs(gp.astype(np.float64) - ref.planes[1].astype(np.float64))
+                assert np.all(err <= 1e-5 * np.maximum(_abs_mass(p, U)[:, :, None, None], 1.0))
+        finally:
+            g.close()
