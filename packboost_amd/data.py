@@ -149,12 +149,15 @@ def feature_names_or_default(feature_names: Sequence[str] | None, n_features: in
 
 
 def _float_matrix_device(X, device):
-    """float32 [N, F] on the device: a row's features adjacent, or a feature's rows."""
+    """float32 [N, F] on the device: a row's features adjacent, or a feature's rows (columns that
+    overlap, as an expanded one's do, are copied out)."""
     import torch
 
     if isinstance(X, torch.Tensor):
         x = X.detach().to(device=device, dtype=torch.float32)
-        return x if x.dim() == 2 and 1 in x.stride() else x.contiguous()
+        if x.dim() == 2 and (x.stride(1) == 1 or (x.stride(0) == 1 and x.stride(1) >= x.shape[0])):
+            return x
+        return x.contiguous()
     Xn = np.asarray(ensure_numpy(X), dtype=np.float32)
     if not (Xn.flags.c_contiguous or Xn.flags.f_contiguous):
         Xn = np.ascontiguousarray(Xn)

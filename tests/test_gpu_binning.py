@@ -158,3 +158,22 @@ def test_column_quantiles(hip, n, nb):
             got.append(bins_fm[:, :n].cpu().numpy().T)
             np.testing.assert_array_equal(got[-1][:, ascends], want_b[:, ascends])
     np.testing.assert_array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("n,f", [(50, 1), (50, 7), (1, 3)])
+def test_overlapping_columns(hip, n, f):
+    """One column seen as several, and windows over one series: their columns overlap in memory."""
+    import torch
+
+    from packboost_amd.data import apply_bins_device, quantile_bin_device
+
+    dev = torch.device("cuda")
+    series = torch.randn(n + f, generator=torch.Generator().manual_seed(n)).to(dev)
+    for x in (series[:n, None].expand(n, f), series.as_strided((n, f), (1, 1)), series[None, :f].expand(n, f)):
+        X = x.cpu().numpy().copy()
+        want_b, want_e = _host_bins(X, 6)
+        got, edges = quantile_bin_device(x, 6, dev)
+        assert_edges_equal(edges, want_e, f"strides {x.stride()}")
+        np.testing.assert_array_equal(got[:, :n].cpu().numpy().T, want_b)
+        again = apply_bins_device(x, want_e, 6, dev)
+        np.testing.assert_array_equal(again[:, :n].cpu().numpy().T, want_b)
