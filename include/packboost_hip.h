@@ -504,11 +504,12 @@ int pb_rowlist_gather(const uint8_t* bins_dev, int64_t N, int64_t ld, int32_t F,
  * (bad_hess), a weight of an era without rows is not 0 (stray_weight), some era has rows (counted)
  * and a weight other than 1 (not_unit), a drawn feature id lies outside [0, F) (bad_feature), a bin
  * of a drawn column is >= limit (bin_over); the least and greatest weight - rows over eras with
- * rows (alpha_lo, alpha_hi: -inf, inf with a NaN weight), and the listed rows of all nodes. bins
+ * rows (negative ones and NaN as 0; alpha_most the bits of the double, alpha_least their complement;
+ * both 0 when no era has rows), and the listed rows of all nodes. bins
  * uint8 [F][ld] (any alignment), weights float32 [M][E], node_era_splits int32 [M][E + 1]. */
 typedef struct pb_rowlist_facts {
     int32_t bad_hess, stray_weight, counted, not_unit, bad_feature, bin_over, reserved[2];
-    double alpha_lo, alpha_hi;
+    uint64_t alpha_least, alpha_most;
     int64_t rows, reserved2;
 } pb_rowlist_facts;
 int pb_rowlist_facts_get(const uint8_t* bins_dev, int64_t N, int64_t ld, int32_t F, const int32_t* feats_dev,

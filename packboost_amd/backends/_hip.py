@@ -90,7 +90,7 @@ CANDIDATE_DTYPE = np.dtype([
 ])
 FACTS_DTYPE = np.dtype([
     ("bad_hess", "<i4"), ("stray_weight", "<i4"), ("counted", "<i4"), ("not_unit", "<i4"), ("bad_feature", "<i4"),
-    ("bin_over", "<i4"), ("reserved", "<i4", (2,)), ("alpha_lo", "<f8"), ("alpha_hi", "<f8"), ("rows", "<i8"),
+    ("bin_over", "<i4"), ("reserved", "<i4", (2,)), ("alpha_least", "<u8"), ("alpha_most", "<u8"), ("rows", "<i8"),
     ("reserved2", "<i8"),
 ])
 assert FACTS_DTYPE.itemsize == 64

@@ -55,9 +55,10 @@ def _era_alpha_of(facts: np.ndarray) -> float:
         raise RuntimeError("era_weights must be 0 for eras without rows")
     if not facts["counted"] or not facts["not_unit"]:
         return 0.0
-    if facts["alpha_lo"] != facts["alpha_hi"] or not facts["alpha_lo"] > 0.0:
+    least, most = (~facts["alpha_least"]).view(np.float64), facts["alpha_most"].view(np.float64)
+    if least != most or not least > 0.0:
         raise RuntimeError("era_weights are not count + era_alpha for one era_alpha > 0")
-    return float(facts["alpha_lo"])
+    return float(most)
 
 
 _STATUS = ("a (node, era) segment lies outside rows_index", "a row id lies outside [0, N)",

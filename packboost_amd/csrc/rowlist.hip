@@ -418,29 +418,31 @@ __global__ __launch_bounds__(kRlBlock) void rl_best_kernel(const pb_candidate* _
 }
 
 // What a call's inputs must satisfy, looked up in one launch (RowlistFacts, cleared by the caller):
-// workgroup 0 covers the weights and row counts, the others hess and the drawn columns' bins.
+// the first `wblocks` workgroups cover the weights and row counts, one (node, era) pair a thread up
+// to 512 workgroups (a single workgroup waited on its loads pair after pair: split search over
+// 1024 x 574 lists and 8 features 2.25 ms, 1.10 so), the others hess and the drawn columns' bins. The least and greatest weight - rows are joined as the
+// bit patterns of non-negative doubles, whose order is the numbers'; the least as its complement, so
+// that a cleared record is the neutral one of both.
 __global__ __launch_bounds__(kRlBlock) void rl_facts_kernel(
     const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F, const int32_t* __restrict__ feats, int32_t K,
     const float* __restrict__ hess, int64_t n_hess, const float* __restrict__ weights, const int32_t* __restrict__ nes,
-    int32_t M, int32_t E, uint32_t limit, pb_rowlist_facts* out) {
+    int32_t M, int32_t E, uint32_t limit, int32_t wblocks, pb_rowlist_facts* out) {
     const int lane = threadIdx.x & (kWave - 1);
-    if (blockIdx.x == 0) {
-        __shared__ double s_lo[kRlWaves], s_hi[kRlWaves];
-        __shared__ unsigned long long s_rows[kRlWaves];
-        double lo = __builtin_inf(), hi = -__builtin_inf();
-        unsigned long long total = 0ull;
+    if ((int)blockIdx.x < wblocks) {
+        unsigned long long least = 0ull, most = 0ull, total = 0ull;
         bool stray = false, counted = false, unit = true;
-        for (int64_t x = threadIdx.x; x < (int64_t)M * E; x += kRlBlock) {
+        for (int64_t x = (int64_t)blockIdx.x * kRlBlock + threadIdx.x; x < (int64_t)M * E;
+             x += (int64_t)wblocks * kRlBlock) {
             const int64_t s = x / E, e = x - s * E;
             const int32_t c = nes[s * (E + 1) + e + 1] - nes[s * (E + 1) + e];
             const float w = weights[x];
             if (c > 0) {
                 const double d = (double)w - (double)c;
+                const unsigned long long key = d > 0.0 ? (unsigned long long)__double_as_longlong(d) : 0ull;  // 0: NaN too
                 counted = true;
                 unit &= w == 1.0f;
-                lo = fmin(lo, d);
-                hi = fmax(hi, d);
-                if (isnan(w)) lo = -__builtin_inf(), hi = __builtin_inf();  // no common era_alpha
+                least = max(least, ~key);
+                most = max(most, key);
             } else {
                 stray |= !(w == 0.0f);
             }
@@ -449,37 +451,27 @@ __global__ __launch_bounds__(kRlBlock) void rl_facts_kernel(
                 total += rows > 0 ? (unsigned long long)rows : 0ull;
             }
         }
-        for (int32_t k = threadIdx.x; k < K; k += kRlBlock)
-            if (feats[k] < 0 || feats[k] >= F) out->bad_feature = 1;
+        if (blockIdx.x == 0)
+            for (int32_t k = threadIdx.x; k < K; k += kRlBlock)
+                if (feats[k] < 0 || feats[k] >= F) out->bad_feature = 1;
         if (stray) out->stray_weight = 1;
         if (counted) out->counted = 1;
         if (!unit) out->not_unit = 1;
 #pragma unroll
         for (int m = 1; m < kWave; m <<= 1) {
-            lo = fmin(lo, __shfl_xor(lo, m));
-            hi = fmax(hi, __shfl_xor(hi, m));
+            least = max(least, (unsigned long long)__shfl_xor(least, m));
+            most = max(most, (unsigned long long)__shfl_xor(most, m));
             total += __shfl_xor(total, m);
         }
         if (lane == 0) {
-            s_lo[threadIdx.x / kWave] = lo;
-            s_hi[threadIdx.x / kWave] = hi;
-            s_rows[threadIdx.x / kWave] = total;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int w = 1; w < kRlWaves; ++w) {
-                lo = fmin(lo, s_lo[w]);
-                hi = fmax(hi, s_hi[w]);
-                total += s_rows[w];
-            }
-            out->alpha_lo = lo;
-            out->alpha_hi = hi;
-            out->rows = (int64_t)total;
+            if (least) atomicMax(reinterpret_cast<unsigned long long*>(&out->alpha_least), least);
+            if (most) atomicMax(reinterpret_cast<unsigned long long*>(&out->alpha_most), most);
+            if (total) atomicAdd(reinterpret_cast<unsigned long long*>(&out->rows), total);
         }
         return;
     }
-    const int64_t t = (int64_t)(blockIdx.x - 1) * kRlBlock + threadIdx.x;
-    const int64_t stride = (int64_t)(gridDim.x - 1) * kRlBlock;
+    const int64_t t = (int64_t)((int)blockIdx.x - wblocks) * kRlBlock + threadIdx.x;
+    const int64_t stride = (int64_t)((int)gridDim.x - wblocks) * kRlBlock;
     bool bad = false;
     for (int64_t i = t; i < n_hess; i += stride) bad |= !(hess[i] == 1.0f);
     if (bad) out->bad_hess = 1;
@@ -625,8 +617,9 @@ hipError_t launch_rowlist_facts(const uint8_t* bins, int64_t N, int64_t ld, int3
                                 const float* hess, int64_t n_hess, const float* weights, const int32_t* nes, int32_t M,
                                 int32_t E, int32_t limit, pb_rowlist_facts* out, hipStream_t s) {
     const int64_t work = std::max<int64_t>(n_hess, (N + 15) / 16 * K);
-    hipLaunchKernelGGL(rl_facts_kernel, dim3(1 + grid_of(work, kRlBlock, 2048)), dim3(kRlBlock), 0, s, bins, N, ld, F,
-                       feats, K, hess, n_hess, weights, nes, M, E, (uint32_t)limit, out);
+    const int32_t wblocks = grid_of((int64_t)M * E, kRlBlock, 512);
+    hipLaunchKernelGGL(rl_facts_kernel, dim3(wblocks + grid_of(work, kRlBlock, 2048)), dim3(kRlBlock), 0, s, bins, N, ld,
+                       F, feats, K, hess, n_hess, weights, nes, M, E, (uint32_t)limit, wblocks, out);
     return hipGetLastError();
 }
 

@@ -412,6 +412,59 @@ def test_split_finder_input_checks(hip, what):
             call()
 
 
+@pytest.mark.parametrize("fault", ["none", "unit", "stray", "alpha", "negative"])
+@pytest.mark.parametrize("nodes,eras", [(1, 1), (3, 200), (7, 37)])
+def test_split_finder_weights_over_workgroups(hip, nodes, eras, fault):
+    """More (node, era) pairs than one workgroup of the device's look at the weights covers, with a
+    fault in the last one: float32 weights (looked at there) and float64 ones (on the host) agree."""
+    import torch
+
+    from packboost_amd import backends
+
+    rng = np.random.default_rng(nodes * 1000 + eras)
+    size = rng.integers(2, 9, (nodes, eras))
+    if eras > 1:
+        size[:, ::5] = 0
+        size[-1, -1] = 0 if fault == "stray" else 3
+    elif fault == "stray":
+        size[:] = 0
+    N, F = int(size.sum()) + 40, 6
+    dev = torch.device("cuda")
+    bins = torch.from_numpy(rng.integers(0, 5, (F, N), dtype=np.uint8)).to(dev)
+    rows = torch.from_numpy(rng.permutation(N)[:size.sum()].astype(np.int32)).to(dev)
+    nes = torch.zeros((nodes, eras + 1), dtype=torch.int32)
+    nes[:, 1:] = torch.from_numpy(size.cumsum(1))
+    nrs = torch.zeros(nodes + 1, dtype=torch.int32)
+    nrs[1:] = torch.from_numpy(size.sum(1).cumsum())
+    grad = torch.from_numpy(rng.standard_normal(int(size.sum()), dtype=np.float32)).to(dev)
+    cnt = torch.from_numpy(size)
+    w = torch.where(cnt > 0, torch.ones(()) if fault == "unit" else cnt + 2.5, torch.zeros(())).float()
+    if fault == "stray":
+        w[-1, -1] = 1.0
+    elif fault == "alpha":
+        w[-1, -1] += 0.5
+    elif fault == "negative":
+        w = torch.where(cnt > 0, cnt - 0.5, torch.zeros(())).float()
+    z = torch.zeros(nodes, device=dev)
+    ids = torch.arange(F, dtype=torch.int32, device=dev)
+
+    def call(weights):
+        try:
+            return backends.find_best_splits_batched_cuda(
+                bins, grad, torch.ones_like(grad), rows, nrs.to(dev), nes.to(dev), weights.to(dev), z, z, z.long(), ids,
+                5, 0, "mass", 1e-3, 0.4, 0.1, 2)
+        except RuntimeError as e:
+            return str(e)
+
+    got, ref = call(w), call(w.double())
+    refused = fault in ("stray", "negative") or (fault == "alpha" and nodes * eras > 1)
+    assert isinstance(got, str) == isinstance(ref, str) == refused
+    if refused:
+        assert got == ref
+    else:
+        assert all(torch.equal(got[k], ref[k]) for k in ("scores", "thresholds", "left_grad", "left_count"))
+
+
 @pytest.mark.parametrize("sizes", [[0], [1], [63, 64, 65], [255, 0, 256, 257], [1000, 3, 511, 512, 513]], ids=str)
 def test_partition_totals(hip, sizes):
     """Segments of 0 to 1000 rows at wavefront edges, and a row id and a feature that are refused:
