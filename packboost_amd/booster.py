@@ -235,6 +235,9 @@ class PackBoost:
         self._trained_pack_size: int | None = None
         self._round_metrics: list[dict[str, float]] = []
         self._packed_forest: list[dict[str, torch.Tensor]] = []
+        # the fitted rounds on the device, packed and compiled, with the key each was made for
+        self._forest_cache: tuple | None = None
+        self._compiled_forest: tuple | None = None
         self._num_features: int | None = None
         self._use_native_cuda = self._device.type == "cuda" and native_backends.cuda_available()
         # per-depth phase times in the depth logs (hist_ms, score_ms, partition_ms): every
@@ -315,6 +318,8 @@ class PackBoost:
         self._rounds = []
         self._trees_cache = None
         self._packed_forest = []
+        self._forest_cache = None  # of the last fit's rounds
+        self._compiled_forest = None
         self._tree_weight = None
         self._trained_pack_size = None
 
@@ -443,7 +448,7 @@ class PackBoost:
     # ---------------------------------------------------------------- internals
     def _forest_device(self, device: torch.device) -> dict[str, torch.Tensor]:
         key = (str(device), len(self._rounds))
-        cached = getattr(self, "_forest_cache", None)
+        cached = self._forest_cache
         if cached is not None and cached[0] == key:
             return cached[1]
         forest = pack_forest(self._rounds, int(self._trained_pack_size or self.config.pack_size), device)
@@ -454,7 +459,7 @@ class PackBoost:
         from .predictor import CompiledForest
 
         key = (str(device), len(self._rounds))
-        cached = getattr(self, "_compiled_forest", None)
+        cached = self._compiled_forest
         if cached is None or cached[0] != key:
             cached = (key, CompiledForest(self._forest_device(device)))
             self._compiled_forest = cached

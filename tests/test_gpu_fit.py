@@ -90,6 +90,37 @@ def test_fit_determinism(hip):
                [(n.feature, n.threshold, n.is_leaf, n.value) for n in tb.nodes]
 
 
+@pytest.mark.parametrize("truncate", [False, True])
+def test_refit_predicts_the_new_rounds(hip, truncate):
+    """A model that has predicted is fitted again to another target over as many rounds: predict()
+    (and, where a non-finite round ends the refit, the training predictions, which come from the
+    kept trees) equal a fresh model's."""
+    from packboost_amd import PackBoost, PackBoostConfig
+
+    rng = np.random.default_rng(8)
+    X = rng.integers(0, 8, (3000, 10)).astype(np.uint8)
+    y = X[:, 5] - rng.standard_normal(3000).astype(np.float32)
+    kw = dict(max_depth=3, max_bins=8, min_samples_leaf=5, random_state=4)
+    # learning_rate x pack_size = 128: the residuals grow ~127x a round, past float32 within 20 rounds
+    cfg = PackBoostConfig(pack_size=64, learning_rate=2.0, **kw) if truncate else PackBoostConfig(pack_size=2, **kw)
+
+    def fit(m):
+        if not truncate:
+            return m.fit(X, y, None, num_rounds=5)
+        with pytest.warns(RuntimeWarning, match="not finite"):
+            return m.fit(X, y, None, num_rounds=60)
+
+    fresh = fit(PackBoost(cfg, nonfinite="truncate"))
+    kept = len(fresh._rounds)
+    m = PackBoost(cfg, nonfinite="truncate").fit(X, 1e-25 * X[:, 0].astype(np.float32), None, num_rounds=kept)
+    assert len(m._rounds) == kept > 2
+    before = m.predict(X)
+    fit(m)
+    assert len(m._rounds) == kept and not np.array_equal(m.predict(X), before)
+    np.testing.assert_array_equal(m.predict(X), fresh.predict(X))
+    np.testing.assert_array_equal(m._train_preds.cpu().numpy(), fresh._train_preds.cpu().numpy())
+
+
 def test_unsorted_eras_and_no_eras(hip, oracle_mod):
     """Interleaved era labels (rows permuted era-major inside fit) and era=None."""
     from packboost_amd import PackBoost, PackBoostConfig
