@@ -326,7 +326,7 @@ int pb_transpose_bins(const uint8_t* src_dev, int64_t n, int64_t row_stride, int
 
 /* quantile_bin's edges (data.py:44-56) of F columns of values in any order: element (r, f) at
  * x_dev[r * row_stride + f * col_stride], one of the two strides 1; q_dev, edges_dev and
- * edge_stride as in pb_quantile_edges, whose edges these are (a zero edge is +0.0). work_dev:
+ * edge_stride as in pb_quantile_edges, whose edges these are (of zeros of both signs -0.0 comes first). work_dev:
  * pb_quantile_work_bytes(n, F, num_q) bytes, 256-byte aligned (-1: n not in [1, 2^30], F not in
  * [1, 65535] or num_q not in [1, 254]). */
 int64_t pb_quantile_work_bytes(int64_t n, int32_t F, int32_t num_q);

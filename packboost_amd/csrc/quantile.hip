@@ -4,7 +4,7 @@
 // A quantile needs two neighbouring order statistics of its column; num_q of them pin at most
 // 2 num_q elements, so a sort (a library segmented sort took 110 ms for 1M x 500, and held the
 // sorted values and 64-bit indices) orders far more than is asked. Here, per column:
-//   keys     the values as unsigned order keys, column-major (-0.0 as +0.0, NaN as the last key);
+//   keys     the values as unsigned order keys, column-major (-0.0 before +0.0, NaN as the last key);
 //            row-major input is transposed through LDS, 256 contiguous bytes each way
 //   sample   a sorted sample's every fourth key gives the splitters (2^STEPS - 1 of them)
 //   count    every key's class by a branchless search in LDS: 2i = strictly between splitters
@@ -32,10 +32,11 @@ constexpr int kTile = 64;          // rows and features of a transposed tile
 constexpr int kChunkKeys = 32768;  // keys per workgroup of the count pass
 constexpr uint32_t kNanKey = 0xffffffffu;
 
+// A total order that keeps every bit of a number: a zero edge has the sign that its ranks' zeros give
+// it. (Where a column holds zeros of both signs, which tie in NumPy's sort, -0.0 comes first.)
 __device__ __forceinline__ uint32_t key_of(float x) {
     const uint32_t b = __float_as_uint(x);
-    const uint32_t k = b == 0x80000000u ? 0x80000000u : b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
-    return isnan(x) ? kNanKey : k;
+    return isnan(x) ? kNanKey : b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
 }
 
 __device__ __forceinline__ float value_of(uint32_t k) {

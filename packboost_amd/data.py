@@ -11,7 +11,8 @@ Bins are returned as uint8 (values identical to the reference's int8 for max_bin
 
 quantile_bin_device / apply_bins_device do the same on the HIP device (pb_column_quantiles,
 pb_bin_rows) and write the histogram kernel's column-major layout directly; their edges and
-bins are bit-identical to the NumPy path.
+bins are bit-identical to the NumPy path (but for a zero edge's sign in a column that mixes -0.0
+and +0.0, which a sort may leave in any order).
 """
 
 from __future__ import annotations

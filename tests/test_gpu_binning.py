@@ -160,6 +160,23 @@ def test_column_quantiles(hip, n, nb):
     np.testing.assert_array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("n", [2, 1003, 16384, 16386, 30_002, 530_002])
+def test_zero_edges_keep_their_sign(hip, n):
+    """Columns whose zeros all have one sign (a rectified column and its negative, and zeros alone):
+    edges equal NumPy's bit for bit, signs of zeros included, sorted in LDS and selected."""
+    import torch
+
+    from packboost_amd.data import quantile_bin_device
+
+    z = np.maximum(np.random.default_rng(n).standard_normal(n), 0).astype(np.float32)
+    X = np.stack([z, -z, np.zeros_like(z), np.full_like(z, -0.0)], axis=1)
+    want = _host_bins(X, 8)[1]
+    assert np.signbit(want[want == 0]).any()
+    for x in (X, np.asfortranarray(X)):
+        edges = quantile_bin_device(x, 8, torch.device("cuda"))[1]
+        np.testing.assert_array_equal(edges.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("n,f", [(50, 1), (50, 7), (1, 3)])
 def test_overlapping_columns(hip, n, f):
     """One column seen as several, and windows over one series: their columns overlap in memory."""
