@@ -91,6 +91,17 @@ __global__ __launch_bounds__(kBlock) void era_corr_mean_kernel(const double* __r
 constexpr int kCorrRows = 16;  // rows per thread
 constexpr int kCorrWin = kBlock * kCorrRows;
 
+// One past the last row of the window that starts at w0 (a multiple of kCorrWin below n): w0 +
+// kCorrWin passes 2^31 - 1 in the last window of the longest tables. Every row of the window, of the
+// last one's lanes too, is then at most w0 + kCorrWin - 1 <= 2^31 - 1.
+__host__ __device__ constexpr int window_end(int w0, int n) { return n - w0 < kCorrWin ? n : w0 + kCorrWin; }
+constexpr int kLastWin = INT32_MAX - (kCorrWin - 1);
+static_assert(kLastWin % kCorrWin == 0 && window_end(kLastWin, INT32_MAX) == INT32_MAX &&
+                  window_end(kLastWin, kLastWin + 1) == kLastWin + 1 &&
+                  window_end(kLastWin - kCorrWin, INT32_MAX) == kLastWin && window_end(0, 1) == 1 &&
+                  window_end(0, kCorrWin) == kCorrWin,
+              "a window ends within the rows, up to 2^31 - 1 of them");
+
 struct Moments {  // of one era's rows in one window
     double n, my, mp, syy, spp, syp;
 };
@@ -119,7 +130,7 @@ __global__ __launch_bounds__(kBlock) void era_corr_windows_kernel(const float* _
                                                               Moments* __restrict__ slots) {
     __shared__ double sh[kBlock / kWave][4];
     const int w0 = blockIdx.x * kCorrWin;
-    const int w1 = min(w0 + kCorrWin, n);
+    const int w1 = window_end(w0, n);
     float yv[kCorrRows], pv[kCorrRows];
 #pragma unroll
     for (int i = 0; i < kCorrRows; ++i) {

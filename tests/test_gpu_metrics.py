@@ -126,6 +126,34 @@ def test_era_corr_rows(hip, sizes):
     np.testing.assert_allclose([out.item(), was[E]], [era_corr_np(era, y, p)] * 2, rtol=0, atol=1e-9)
 
 
+@pytest.mark.parametrize("n", [2**31 - 1, 2**31 - 4095, 2**31 - 4096])
+def test_era_corr_rows_to_the_last_row(hip, n):
+    """The longest tables pb_era_corr_rows takes: one era whose last rows alone vary, so its
+    correlation comes from the last windows of rows (and their ends near 2^31)."""
+    import torch
+
+    from packboost_amd.booster import _corr_scratch, _era_corr_enqueue
+
+    dev = torch.device("cuda")
+    if torch.cuda.mem_get_info(dev)[0] < 24 << 30:
+        pytest.skip("needs 24 GiB of device memory")
+    tail = 3000
+    rng = np.random.default_rng(5)
+    yt = rng.standard_normal(tail).astype(np.float32)
+    pt = (yt + rng.standard_normal(tail)).astype(np.float32)
+    y, p = torch.zeros(n, device=dev), torch.zeros(n, device=dev)
+    y[n - tail:], p[n - tail:] = torch.from_numpy(yt), torch.from_numpy(pt)
+    off = torch.tensor([0, n], dtype=torch.int32, device=dev)
+    scratch = _corr_scratch(n, 1, dev).zero_()
+    out = torch.empty(1, dtype=torch.float64, device=dev)
+    _era_corr_enqueue(y, p, off, scratch, out)
+    yd, pd_ = yt.astype(np.float64), pt.astype(np.float64)
+    my, mp = yd.sum() / n, pd_.sum() / n  # of all rows; those before the tail are zero
+    syy, spp, syp = ((a * b).sum() - n * ma * mb for a, b, ma, mb in
+                     ((yd, yd, my, my), (pd_, pd_, mp, mp), (yd, pd_, my, mp)))
+    np.testing.assert_allclose(out.item(), syp / np.sqrt(syy * spp), rtol=0, atol=1e-9)
+
+
 @pytest.mark.parametrize("depth,B", [(0, 3), (1, 1), (6, 8), (9, 2), (10, 5)])
 def test_fold_tree(hip, depth, B):
     """pb_fold_tree (records in LDS up to 1024 nodes, in memory above) against pb_predict_bins and
