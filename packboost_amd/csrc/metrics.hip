@@ -45,7 +45,7 @@ __global__ __launch_bounds__(kBlock) void era_corr_kernel(const float* __restric
     const int r0 = era_off[e], r1 = era_off[e + 1];
     const int n = r1 - r0;
     double sy = 0.0, sp = 0.0;
-    for (int r = r0 + (int)threadIdx.x; r < r1; r += kBlock) {
+    for (int64_t r = (int64_t)r0 + threadIdx.x; r < r1; r += kBlock) {  // past 2^31 at the last rows
         sy += (double)y[r];
         sp += (double)p[r];
     }
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kBlock) void era_corr_kernel(const float* __restric
     sp = block_sum(sp, sh);
     const double my = n > 0 ? sy / n : 0.0, mp = n > 0 ? sp / n : 0.0;
     double syy = 0.0, spp = 0.0, syp = 0.0;
-    for (int r = r0 + (int)threadIdx.x; r < r1; r += kBlock) {
+    for (int64_t r = (int64_t)r0 + threadIdx.x; r < r1; r += kBlock) {
         const double dy = (double)y[r] - my, dp = (double)p[r] - mp;
         syy += dy * dy;
         spp += dp * dp;

@@ -128,8 +128,9 @@ def test_era_corr_rows(hip, sizes):
 
 @pytest.mark.parametrize("n", [2**31 - 1, 2**31 - 4095, 2**31 - 4096])
 def test_era_corr_rows_to_the_last_row(hip, n):
-    """The longest tables pb_era_corr_rows takes: one era whose last rows alone vary, so its
-    correlation comes from the last windows of rows (and their ends near 2^31)."""
+    """The longest tables the era correlations take: one era whose last rows alone vary, so its
+    correlation comes from the last windows of rows, and an era of those rows (row numbers up to
+    2^31 - 1, which a step of 256 rows passes)."""
     import torch
 
     from packboost_amd.booster import _corr_scratch, _era_corr_enqueue
@@ -147,6 +148,11 @@ def test_era_corr_rows_to_the_last_row(hip, n):
     scratch = _corr_scratch(n, 1, dev).zero_()
     out = torch.empty(1, dtype=torch.float64, device=dev)
     _era_corr_enqueue(y, p, off, scratch, out)
+    # the tail as an era of its own, by pb_era_corr's workgroup per era
+    ends, each = torch.tensor([n - tail, n], dtype=torch.int32, device=dev), torch.empty(2, dtype=torch.float64, device=dev)
+    hip.check(hip.load().pb_era_corr(y.data_ptr(), p.data_ptr(), ends.data_ptr(), 1, each.data_ptr(),
+                                     each.data_ptr() + 8, hip.stream_ptr()), "pb_era_corr")
+    np.testing.assert_allclose(each.cpu().numpy(), [era_corr_np(np.zeros(tail), yt, pt)] * 2, rtol=0, atol=1e-9)
     yd, pd_ = yt.astype(np.float64), pt.astype(np.float64)
     my, mp = yd.sum() / n, pd_.sum() / n  # of all rows; those before the tail are zero
     syy, spp, syp = ((a * b).sum() - n * ma * mb for a, b, ma, mb in
