@@ -66,8 +66,11 @@ _STATUS = ("a (node, era) segment lies outside rows_index", "a row id lies outsi
 
 
 def _facts(lib, b_fm, F, N, ld, fid, K, hess, weights, nes, M, E, limit) -> np.ndarray:
-    """pb_rowlist_facts of the call's inputs: one launch and one wait."""
+    """pb_rowlist_facts of the call's inputs: one launch and one wait. Columns that overlap (one seen
+    as several, windows over a series) are looked at in a copy."""
     dev = b_fm.device
+    if ld < N:
+        b_fm, ld = b_fm.clone(memory_format=torch.contiguous_format), N
     out = torch.zeros(_hip.FACTS_DTYPE.itemsize, dtype=torch.uint8, device=dev)
     h = hess.to(device=dev, dtype=torch.float32).contiguous()
     _hip.check(lib.pb_rowlist_facts_get(b_fm.data_ptr(), N, ld, F, fid.data_ptr(), K, h.data_ptr(), int(h.numel()),

@@ -412,6 +412,36 @@ def test_split_finder_input_checks(hip, what):
             call()
 
 
+@pytest.mark.parametrize("what", ["expanded", "windows", "one_column"])
+def test_split_finder_overlapping_columns(hip, what):
+    """Bins whose columns overlap in memory, some of them above max_bins: the same splits as from a
+    copy of the bins (where none is above, the gather refuses the stride, as it always has)."""
+    import torch
+
+    from packboost_amd import backends
+
+    dev = torch.device("cuda")
+    N = 700
+    series = torch.randint(0, 7, (N + 3,), dtype=torch.uint8, device=dev, generator=torch.Generator("cuda").manual_seed(3))
+    bins = {"expanded": series[None, :N].expand(3, N), "windows": series.as_strided((3, N), (1, 1)),
+            "one_column": series[:N, None].t()}[what]
+    rows = torch.randperm(N).to(device=dev, dtype=torch.int32)
+    grad = torch.randn(N, device=dev)
+    nrs, nes = torch.tensor([0, N], dtype=torch.int32), torch.tensor([[0, N // 2, N]], dtype=torch.int32)
+    z = torch.zeros(1, device=dev)
+    ids = torch.arange(bins.shape[0], dtype=torch.int32, device=dev)
+
+    def call(b, nb):
+        return backends.find_best_splits_batched_cuda(b, grad, torch.ones_like(grad), rows, nrs, nes, torch.ones((1, 2)),
+                                                      z, z, z.long(), ids, nb, 0, "mass", 1e-3, 0.4, 0.1, 5)
+
+    got, want = call(bins, 5), call(bins.clone(memory_format=torch.contiguous_format), 5)
+    for key in ("scores", "thresholds", "left_grad", "left_hess", "left_count"):
+        assert torch.equal(got[key], want[key])
+    with pytest.raises(hip.HipBackendError, match="N must be <= ld"):
+        call(bins, 8)
+
+
 @pytest.mark.parametrize("fault", ["none", "unit", "stray", "alpha", "negative"])
 @pytest.mark.parametrize("nodes,eras", [(1, 1), (3, 200), (7, 37)])
 def test_split_finder_weights_over_workgroups(hip, nodes, eras, fault):
