@@ -501,8 +501,8 @@ class PackBoost:
         # same rows: the sum over every tree so far, in tree order, of float32(weight * value).
         # That sum is a left fold, so each state extends its own fold by the rounds it has not
         # seen, one float32 add per tree: the B trees of a round are identical, so the round's
-        # tree is walked once (pb_predict_bins) and its weighted value added B times. The host
-        # work per eval is the new rounds only.
+        # tree is walked once and its weighted value added B times, in place (pb_fold_tree). The
+        # host work per eval is the new rounds only.
         B = int(self.config.pack_size)
         lib = _hip.load()
         trees: dict[int, torch.Tensor] = {}
@@ -519,8 +519,11 @@ class PackBoost:
 
 
 def _tree_records(a: dict[str, np.ndarray]) -> np.ndarray:
-    """One tree's arrays as pb_fold_tree's node records, int32 [nodes, 4] (a split's right child
-    follows its left one, as TreeBuilder numbers them)."""
+    """One tree's arrays as pb_fold_tree's node records, int32 [nodes, 4]. A record names its left
+    child alone: the right one must follow it, as TreeBuilder numbers them."""
+    split = ~np.asarray(a["is_leaf"], dtype=bool)
+    if np.any(np.asarray(a["right"])[split] != np.asarray(a["left"])[split] + 1):
+        raise ValueError("pb_fold_tree needs every split's right child next to its left one")
     rec = np.empty((len(a["feature"]), 4), dtype=np.int32)
     rec[:, 0] = np.where(a["is_leaf"], -1, a["feature"])
     rec[:, 1] = a["threshold"]

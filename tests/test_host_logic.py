@@ -36,6 +36,26 @@ def test_encode_eras_and_era_major_order():
     np.testing.assert_array_equal(offs2, [0, 2, 5])
 
 
+def test_tree_records():
+    """The records of the validation sets' tree walk: feature (-1: leaf), threshold, left child, value
+    bits; a tree whose right child does not follow the left one is refused, since the record does
+    not hold it."""
+    from packboost_amd.booster import _tree_records
+
+    tree = {"feature": np.array([3, -1, 1, -1, -1]), "threshold": np.array([7, -1, 2, -1, -1]),
+            "left": np.array([1, -1, 3, -1, -1]), "right": np.array([2, -1, 4, -1, -1]),
+            "value": np.array([0.0, 0.5, 0.0, -2.0, 1e-3]), "is_leaf": np.array([False, True, False, True, True])}
+    rec = _tree_records(tree)
+    assert rec.dtype == np.int32 and rec.shape == (5, 4)
+    np.testing.assert_array_equal(rec[:, 0], [3, -1, 1, -1, -1])
+    np.testing.assert_array_equal(rec[[0, 2], 1:3], [[7, 1], [2, 3]])
+    np.testing.assert_array_equal(rec[:, 3].view(np.float32), tree["value"].astype(np.float32))
+    _tree_records({k: v[1:2] for k, v in tree.items()})  # a leaf alone
+    swapped = dict(tree, left=np.array([2, -1, 3, -1, -1]), right=np.array([1, -1, 4, -1, -1]))
+    with pytest.raises(ValueError, match="right child"):
+        _tree_records(swapped)
+
+
 def test_subset_size_rule():
     from packboost_amd import PackBoostConfig
     from packboost_amd.engine import subset_size
