@@ -72,12 +72,14 @@ __global__ __launch_bounds__(kBlock) void predict_pack_kernel(
 
 // predict_pack_kernel for forests of up to kPackNodes nodes: the nodes sit in LDS as 16-byte records
 // (feature, or -1 for a leaf with its value bits in the next word; threshold; children) and a lane
-// walks 8 trees a level at a time, so that their bin loads are in flight together. The one-tree
-// walk waited on a node and a bin in turn, 48 times in a row for 8 trees of depth 6:
-// 188 us for 600k rows, 54 us so (about the bytes of the columns it reads at the copy rate).
+// walks TREES trees a level at a time, so that their bin loads are in flight together. The one-tree
+// walk waited on a node and a bin in turn, 48 times in a row for 8 trees of depth 6: 108 us for 600k
+// rows of 1200 features, 43 us so. A place in the group without a tree costs as much as one with: two
+// trees in groups of eight took 63 us for 2M rows at depth 6 (40 at depth 3), 44 (27) in groups of two,
+// 66 (29) one after the other.
 constexpr int kPackNodes = 2048;
-constexpr int kPackTrees = 8;
 
+template <int TREES>
 __global__ __launch_bounds__(kBlock) void predict_pack_lds_kernel(
     const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F, const int32_t* __restrict__ feature,
     const int32_t* __restrict__ threshold, const int32_t* __restrict__ left_abs, const int32_t* __restrict__ right_abs,
@@ -94,12 +96,12 @@ __global__ __launch_bounds__(kBlock) void predict_pack_lds_kernel(
     const int64_t stride = (int64_t)gridDim.x * kBlock;
     for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < N; r += stride) {
         float s = 0.0f;
-        for (int t0 = 0; t0 < B; t0 += kPackTrees) {
-            int32_t node[kPackTrees], lo[kPackTrees], hi[kPackTrees], lf[kPackTrees];
-            float v[kPackTrees];
+        for (int t0 = 0; t0 < B; t0 += TREES) {
+            int32_t node[TREES], lo[TREES], hi[TREES], lf[TREES];
+            float v[TREES];
             int32_t steps = 0;
 #pragma unroll
-            for (int j = 0; j < kPackTrees; ++j) {
+            for (int j = 0; j < TREES; ++j) {
                 // a tree's span, clamped to the node arrays (offsets come from the caller)
                 const int t = min(t0 + j, B - 1);
                 lo[j] = min(max(offsets[t], 0), total_nodes);
@@ -110,16 +112,16 @@ __global__ __launch_bounds__(kBlock) void predict_pack_lds_kernel(
                 steps = max(steps, hi[j] - lo[j]);
             }
             for (int it = 0; it < steps; ++it) {
-                int4 q[kPackTrees];
-                int32_t bin[kPackTrees];
+                int4 q[TREES];
+                int32_t bin[TREES];
 #pragma unroll
-                for (int j = 0; j < kPackTrees; ++j) q[j] = s_node[max(node[j], 0)];
+                for (int j = 0; j < TREES; ++j) q[j] = s_node[max(node[j], 0)];
 #pragma unroll
-                for (int j = 0; j < kPackTrees; ++j)  // in bounds whatever the record
+                for (int j = 0; j < TREES; ++j)  // in bounds whatever the record
                     bin[j] = bins[(int64_t)max(q[j].x, 0) * ld + r];
                 bool live = false;
 #pragma unroll
-                for (int j = 0; j < kPackTrees; ++j) {
+                for (int j = 0; j < TREES; ++j) {
                     if (node[j] < 0) continue;
                     const int32_t next = bin[j] <= q[j].y ? q[j].z : q[j].w;
                     if (q[j].x == -1) {
@@ -133,7 +135,7 @@ __global__ __launch_bounds__(kBlock) void predict_pack_lds_kernel(
                 if (!live) break;
             }
 #pragma unroll
-            for (int j = 0; j < kPackTrees; ++j) {
+            for (int j = 0; j < TREES; ++j) {
                 if (t0 + j >= B) continue;
                 s = sequential ? (s + tree_weight * v[j]) : (s + v[j]);
                 if (leaf) leaf[(int64_t)(t0 + j) * N + r] = lf[j];
@@ -590,13 +592,16 @@ hipError_t launch_predict_pack(const uint8_t* bins, int64_t N, int64_t ld, int32
                                const int32_t* offsets, int32_t B, int32_t total_nodes,
                                float tree_weight, int32_t sequential, float* out, int32_t* leaf,
                                hipStream_t s) {
-    // the LDS walk while the forest fits its records (about 16 depth-6 trees); a longer forest's nodes
-    // are read where they lie
-    if (total_nodes > 0 && total_nodes <= kPackNodes) {
-        hipLaunchKernelGGL(predict_pack_lds_kernel, dim3(grid_rows(N)), dim3(kBlock), 0, s, bins, N, ld, F, feature,
-                           threshold, left_abs, right_abs, value, is_leaf, offsets, B, total_nodes, tree_weight,
-                           sequential, out, leaf);
-        return hipGetLastError();
+    // the LDS walk from two trees on, while the forest fits its records (about 16 depth-6 trees); a longer
+    // forest's nodes are read where they lie, and so are one tree's, which has no second load to wait
+    // with (2M rows, depths 1 / 3 / 6: 9 / 16 / 41 us, staged and walked in a group of eight 24 / 32 / 57)
+    if (B >= 2 && total_nodes > 0 && total_nodes <= kPackNodes) {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(grid_rows(N)), dim3(kBlock), 0, s, bins, N, ld, F, feature, threshold, left_abs,
+                               right_abs, value, is_leaf, offsets, B, total_nodes, tree_weight, sequential, out, leaf);
+            return hipGetLastError();
+        };
+        return B == 2 ? go(predict_pack_lds_kernel<2>) : go(predict_pack_lds_kernel<8>);
     }
     hipLaunchKernelGGL(predict_pack_kernel, dim3(grid_rows(N)), dim3(kBlock), 0, s, bins, N, ld,
                        F, feature, threshold, left_abs, right_abs, value, is_leaf, offsets, B,

@@ -91,12 +91,14 @@ def test_predict_pack_empty_and_errors(hip):
         np.testing.assert_array_equal(got.cpu().numpy(), second_only.cpu().numpy())
 
 
-@pytest.mark.parametrize("B,D", [(1, 0), (7, 3), (8, 6), (9, 6), (16, 6), (17, 6), (3, 9), (2, 10)])
+@pytest.mark.parametrize("B,D", [(1, 0), (1, 6), (2, 0), (2, 6), (7, 3), (8, 6), (9, 6), (16, 6), (17, 6), (3, 9),
+                                 (2, 10)])
 @pytest.mark.parametrize("view", ["odd", "slice", "columns", "int64"])
 def test_pack_shapes(hip, B, D, view):
-    """The LDS walk (up to 2048 nodes) and the walk in memory (17 trees of depth 6, 2 of depth 10),
-    part-filled groups of trees, odd strides, views and converted inputs: each tree alone through
-    predict_bins_cuda, added in tree order in float32, gives the same sum bit for bit."""
+    """The LDS walk (from two trees on, up to 2048 nodes) and the walk in memory (one tree, 17 trees of
+    depth 6, 2 of depth 10), groups of two and part-filled groups of eight trees, odd strides, views
+    and converted inputs: each tree alone through predict_bins_cuda, added in tree order in float32,
+    gives the same sum bit for bit."""
     import torch
 
     from packboost_amd.backends import predict_bins_cuda, predict_pack_cuda
