@@ -369,8 +369,8 @@ __global__ void rl_era_off_kernel(const int32_t* scan, int32_t Mc, int32_t E, in
 // (score within 1e-12 of the best: the larger left count, then the larger threshold wins; a
 // non-finite best leaves threshold -1 and zero sums). One wavefront each: 64 candidate records are
 // loaded together and the pick runs over them in order on values every lane reads from the lane
-// that holds them (the rule is not transitive, so the order is kept); a lane walking its own
-// 127 records of 32 bytes waited on each (72 us for 16 x 100, 16 us so).
+// that holds them (the rule is not transitive, so the order is kept). 16 x 100 picks of 127 records:
+// 16 us, where rl_best_lane_kernel waits on each record in turn, 40 us.
 __global__ __launch_bounds__(kRlBlock) void rl_best_kernel(const pb_candidate* __restrict__ cand, int64_t MK, int32_t T,
                                                         float* __restrict__ score, int32_t* __restrict__ thr,
                                                         float* __restrict__ left_grad, float* __restrict__ left_hess,
@@ -415,6 +415,54 @@ __global__ __launch_bounds__(kRlBlock) void rl_best_kernel(const pb_candidate* _
     left_grad[i] = blg;
     left_hess[i] = (float)(int64_t)bl;  // squared loss: hess == 1 per row
     left_count[i] = bl;
+}
+
+// The same pick by one lane, 64 picks to a wavefront.
+__global__ __launch_bounds__(kRlBlock) void rl_best_lane_kernel(const pb_candidate* __restrict__ cand, int64_t MK,
+                                                             int32_t T, float* __restrict__ score,
+                                                             int32_t* __restrict__ thr, float* __restrict__ left_grad,
+                                                             float* __restrict__ left_hess,
+                                                             int64_t* __restrict__ left_count) {
+    const int64_t i = (int64_t)blockIdx.x * kRlBlock + threadIdx.x;
+    if (i >= MK) return;
+    float bs = -__builtin_inff(), blg = 0.0f;
+    int32_t bt = -1;
+    int64_t bl = 0;
+    for (int t = 0; t < T; ++t) {
+        const pb_candidate c = cand[i * T + t];
+        if (!c.valid) continue;
+        const float sc = c.score;
+        const int64_t lc = c.left_total;
+        bool better = sc > bs;
+        if (!better && fabsf(sc - bs) <= 1e-12f) better = lc > bl || (lc == bl && c.threshold > bt);
+        if (better) {
+            bs = sc;
+            bt = c.threshold;
+            blg = c.left_grad;
+            bl = lc;
+        }
+    }
+    if (!(bs == bs) || isinf(bs)) {
+        bt = -1;
+        blg = 0.0f;
+        bl = 0;
+    }
+    score[i] = bs;
+    thr[i] = bt;
+    left_grad[i] = blg;
+    left_hess[i] = (float)bl;  // squared loss: hess == 1 per row
+    left_count[i] = bl;
+}
+
+// A lane a pick where that leaves no wait uncovered: few records each, or enough picks to fill the chip,
+// where a wavefront each would leave most of its lanes idle. T = 4: equal up to 32768 picks, 262144 in
+// 11 us by lanes against 46 by wavefronts; T = 31: 8192 in 11.4 against 8.7, 16384 in 11.4 against
+// 14.2; T = 62: 16384 in 31 against 25, 65536 in 36 against 84; T = 127: 32768 in 82 against 88. Records
+// past the caches go to wavefronts, which read them side by side: 587776 x 15 in 220 against 256,
+// 262144 x 127 in 646 against 1529.
+bool pick_by_lane(int64_t MK, int32_t T) {
+    const int64_t records = MK * T;
+    return T < 48 ? (T <= 16 || MK >= 12288) && records <= 1 << 23 : MK >= 24576 && records <= 1 << 24;
 }
 
 // What a call's inputs must satisfy, looked up in one launch (RowlistFacts, cleared by the caller):
@@ -607,9 +655,11 @@ hipError_t launch_best_thresholds(const pb_candidate* cand, int32_t M, int32_t K
                                   float* score, int32_t* thr, float* left_grad, float* left_hess,
                                   int64_t* left_count, hipStream_t s) {
     const int64_t n = (int64_t)M * K;
-    if ((n + kRlWaves - 1) / kRlWaves > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(rl_best_kernel, dim3((unsigned)((n + kRlWaves - 1) / kRlWaves)), dim3(kRlBlock), 0, s, cand, n,
-                       T, score, thr, left_grad, left_hess, left_count);
+    const bool lanes = pick_by_lane(n, T);
+    const int64_t grid = std::max<int64_t>(1, (n + (lanes ? kRlBlock : kRlWaves) - 1) / (lanes ? kRlBlock : kRlWaves));
+    if (grid > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(lanes ? rl_best_lane_kernel : rl_best_kernel, dim3((unsigned)grid), dim3(kRlBlock), 0, s, cand, n, T,
+                       score, thr, left_grad, left_hess, left_count);
     return hipGetLastError();
 }
 

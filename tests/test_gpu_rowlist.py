@@ -323,11 +323,14 @@ def test_best_thresholds_tie_break(hip):
     assert got_t[1, 2] == -1
 
 
-@pytest.mark.parametrize("nb,T", [(5, 4), (64, 63), (65, 64), (129, 128), (200, 199)])
-def test_best_thresholds_order(hip, nb, T):
+@pytest.mark.parametrize("nb,T,copies", [
+    (5, 4, 1), (5, 4, 50), (17, 16, 1), (18, 17, 1), (18, 17, 586), (48, 47, 585), (48, 47, 586), (49, 48, 1170),
+    (49, 48, 1171), (64, 63, 1), (65, 64, 1), (65, 64, 1171), (129, 128, 1), (200, 199, 1)])
+def test_best_thresholds_order(hip, nb, T, copies):
     """The per-(node, feature) pick over thresholds that tie, nearly tie (within 1e-12, where the
-    scan's order decides), are invalid or infinite, at every record window edge, against the scan
-    in Python: exact."""
+    scan's order decides), are invalid or infinite, at every record window edge, a wavefront and a
+    lane a pick (the features repeated up to either side of the counts that change over), against
+    the scan in Python: exact."""
     import torch
 
     rng = np.random.default_rng(nb)
@@ -343,12 +346,15 @@ def test_best_thresholds_order(hip, nb, T):
     rec["threshold"] = rng.permutation(T)[None, None, :]
     rec["valid"] = rng.random((M, K, T)) < 0.8
     rec["valid"][0, 0] = 0
-    cand = torch.from_numpy(rec.view(np.uint8).reshape(-1)).cuda()
-    s, g, h = (torch.empty((M, K), dtype=torch.float32, device="cuda") for _ in range(3))
-    t = torch.empty((M, K), dtype=torch.int32, device="cuda")
-    c = torch.empty((M, K), dtype=torch.int64, device="cuda")
-    hip.check(hip.load().pb_best_thresholds(cand.data_ptr(), M, K, T, s.data_ptr(), t.data_ptr(), g.data_ptr(),
+    wide = K * copies
+    cand = torch.from_numpy(rec.view(np.uint8).reshape(M, K, -1)).cuda().repeat(1, copies, 1)
+    s, g, h = (torch.empty((M, wide), dtype=torch.float32, device="cuda") for _ in range(3))
+    t = torch.empty((M, wide), dtype=torch.int32, device="cuda")
+    c = torch.empty((M, wide), dtype=torch.int64, device="cuda")
+    hip.check(hip.load().pb_best_thresholds(cand.data_ptr(), M, wide, T, s.data_ptr(), t.data_ptr(), g.data_ptr(),
                                             h.data_ptr(), c.data_ptr(), hip.stream_ptr()), "pb_best_thresholds")
+    for out in (s, t, g, h, c):
+        assert torch.equal(out.view(torch.uint8), out[:, :K].repeat(1, copies).view(torch.uint8))
     for m in range(M):
         for k in range(K):
             bs, bt, bg, bl = np.float32(-np.inf), -1, np.float32(0), 0
