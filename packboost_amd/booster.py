@@ -28,7 +28,7 @@ from .config import PackBoostConfig
 from .data import (BinningResult, apply_bins, apply_bins_device, detect_prebinned, encode_eras,
                    era_major_order, feature_names_or_default, preprocess_features,
                    quantile_bin_device)
-from .engine import (DeviceFit, column_major_bins, depth_log_from_round, padded_rows,
+from .engine import (DeviceFit, column_major_bins, depth_log_from_round, features_adjacent, padded_rows,
                      subset_size, transpose_rows, tree_arrays_from_log)
 
 
@@ -132,10 +132,13 @@ def _to_column_major(bins, device: torch.device) -> torch.Tensor:
     """Row-major integer bins [N, F] (numpy or torch) -> contiguous uint8 [F, ld] on device."""
     t = _u8_rows(bins, device)
     N, F = t.shape
-    out = torch.empty((int(F), padded_rows(int(N))), dtype=torch.uint8, device=device)
-    if not transpose_rows(t, out):
+    shape = (int(F), padded_rows(int(N)))
+    if features_adjacent(t):
+        out = torch.empty(shape, dtype=torch.uint8, device=device)
+        transpose_rows(t, out)
+    else:
+        out = torch.zeros(shape, dtype=torch.uint8, device=device)
         out[:, :N] = t.t()
-        out[:, N:] = 0
     return out
 
 
@@ -177,7 +180,7 @@ def _forest_predict(forest, X, bin_edges, max_bins: int, device: torch.device, t
     without a tiled walk go through column-major bins."""
     if not (bin_edges is not None and _is_float_input(X)):
         rows = _u8_rows(_integer_bins(X, bin_edges, max_bins), device)
-        if forest.takes_rows() and (rows.shape[1] == 1 or rows.stride(1) == 1):
+        if features_adjacent(rows) and forest.takes_rows():
             return forest.predict_rows(rows, tree_weight, leaves)
         return forest.predict(_to_column_major(rows, device), int(rows.shape[0]), tree_weight, leaves)
     bins_fm, n = _bins_fm_for(X, bin_edges, max_bins, device)

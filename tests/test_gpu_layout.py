@@ -30,7 +30,8 @@ def test_transpose_bins(hip, n, F, gather):
 
 @pytest.mark.parametrize("limit", [1, 5, 127, 128, 129, 200, 255])
 def test_bin_limit(hip, limit):
-    """One code at the limit is refused wherever it sits; all below it pass."""
+    """One code at the limit is refused wherever it sits, in row-major, feature-major and host tables
+    (each checked on its own route); all below it pass."""
     import torch
 
     from packboost_amd.engine import column_major_bins
@@ -39,10 +40,14 @@ def test_bin_limit(hip, limit):
     n, F = 300, 150
     ok = torch.randint(0, limit, (n, F), dtype=torch.uint8, device=dev)
     ok[0, 0] = limit - 1
-    column_major_bins(ok, None, dev, limit=limit)
+    layouts = (lambda x: x, lambda x: x.t().contiguous().t(), lambda x: x.cpu().numpy(),
+               lambda x: np.asfortranarray(x.cpu().numpy()))
+    for lay in layouts:
+        column_major_bins(lay(ok), None, dev, chunk_rows=128, limit=limit)
     for r, f in ((0, 0), (299, 149), (255, 128), (256, 127), (37, 3)):
         for code in {limit, 255}:
             bad = ok.clone()
             bad[r, f] = code
-            with pytest.raises(ValueError, match="max_bins"):
-                column_major_bins(bad, None, dev, limit=limit)
+            for lay in layouts:
+                with pytest.raises(ValueError, match="max_bins"):
+                    column_major_bins(lay(bad), None, dev, chunk_rows=128, limit=limit)
