@@ -613,6 +613,18 @@ def _same_device(a: torch.device, b: torch.device) -> bool:
     return a.type == b.type and a.index == (torch.cuda.current_device() if b.index is None else b.index)
 
 
+def empty_columns(F: int, N: int, device: torch.device) -> torch.Tensor:
+    """Column-major uint8 [F, ld] for N rows to be written; the padding rows are 0 (a small buffer is
+    cleared whole, which takes one call instead of three)."""
+    ld = padded_rows(N)
+    if ld > N and F * ld <= 1 << 20:
+        return torch.zeros((F, ld), dtype=torch.uint8, device=device)
+    out = torch.empty((F, ld), dtype=torch.uint8, device=device)
+    if ld > N:
+        out[:, N:] = 0
+    return out
+
+
 def features_adjacent(rows: torch.Tensor) -> bool:
     return rows.shape[1] <= 1 or rows.stride(1) == 1
 
@@ -638,9 +650,14 @@ def column_major_bins(bins_rowmajor: np.ndarray | torch.Tensor, perm: np.ndarray
 
     A tensor on the device whose features are adjacent is transposed where it lies, its bins checked
     on the way. Other inputs go through the device in row chunks, so host memory holds only the input;
-    chunks whose features are not adjacent are copied, and their greatest bin is looked for in the
-    result (a table that is feature-major already is a plain copy so: 3M x 16 with the check take
+    chunks whose features are not adjacent, or few, are copied, and the greatest bin is looked for in
+    the result (a table that is feature-major already is a plain copy so: 3M x 16 with the check take
     142 us, 378 with the strided chunks checked).
+
+    pb_transpose_bins works on 16 features of a row at a time, so long tables of 7 to 15 of them are
+    copied where no row gather goes with it (3M x 12: 132 against 148 us, 300k x 12: 46 against 45;
+    3M x 4: 116 against 106; with a gather 300k x 12: 183 against 168), and of host chunks, whose
+    upload takes the longest, up to 31 (300k x 12: 196 against 220 us; x 64: 662 against 630).
     """
     src = bins_rowmajor if isinstance(bins_rowmajor, torch.Tensor) else np.asarray(bins_rowmajor)
     N, F = src.shape
@@ -649,13 +666,14 @@ def column_major_bins(bins_rowmajor: np.ndarray | torch.Tensor, perm: np.ndarray
     perm_t = None if perm is None else torch.as_tensor(perm, dtype=torch.int64)
     over, copied = None, False
     if (isinstance(src, torch.Tensor) and src.is_cuda and _same_device(src.device, device)
-            and src.element_size() == 1 and features_adjacent(src)):
+            and src.element_size() == 1 and features_adjacent(src) and (
+                perm is not None or N < 1 << 20 or not 6 < F < 16)):
         out = torch.empty((F, ld), dtype=torch.uint8, device=device)
         over = torch.zeros(1, dtype=torch.int32, device=device) if check else None
         transpose_rows(src.view(torch.uint8), out, perm=None if perm_t is None else perm_t.to(device), limit=check,
                        over=over)
     else:
-        out = torch.zeros((F, ld), dtype=torch.uint8, device=device)
+        out = empty_columns(F, N, device)
         for r0 in range(0, N, chunk_rows):
             r1 = min(N, r0 + chunk_rows)
             if perm_t is None:
@@ -664,7 +682,7 @@ def column_major_bins(bins_rowmajor: np.ndarray | torch.Tensor, perm: np.ndarray
                 idx = perm_t[r0:r1]
                 part = src[idx.numpy()] if isinstance(src, np.ndarray) else src[idx.to(src.device)]
             t = torch.as_tensor(part).to(device=device).view(torch.uint8)
-            if chunk_rows % 16 == 0 and t.shape[1] == F and features_adjacent(t):
+            if F >= 32 and chunk_rows % 16 == 0 and t.shape[1] == F and features_adjacent(t):
                 if check and over is None:
                     over = torch.zeros(1, dtype=torch.int32, device=device)
                 transpose_rows(t, out, r0, limit=check, over=over)

@@ -171,3 +171,27 @@ def test_rows_walk(hip, D, F, max_thr, N):
         with pytest.raises(hip.HipBackendError, match="feature >= F"):
             cf.predict_rows(wide[:, :top], 0.5)
     cf.close()
+
+
+@pytest.mark.parametrize("n,F", [(300, 1), (300, 9), ((1 << 18) - 1, 9), (1 << 18, 1), (1 << 18, 15), (1 << 18, 16),
+                                 ((1 << 18) + 5, 7)])
+def test_narrow_rows(hip, n, F):
+    """Integer bins of few features, from either side of the counts that send them through
+    column-major bins: the same predictions and leaves as the column-major walk, bit for bit."""
+    import torch
+
+    from packboost_amd.booster import _forest_predict, pack_forest
+    from packboost_amd.engine import padded_rows
+    from packboost_amd.predictor import CompiledForest
+
+    dev = torch.device("cuda")
+    rounds = _forest(n + F, 6, 2, 5, F, ragged=True, max_thr=20)
+    cf = CompiledForest(pack_forest(rounds, 2, dev))
+    rows = torch.randint(0, 24, (n, F + 2), dtype=torch.uint8, device=dev)[:, 1:1 + F]
+    cols = torch.zeros((F, padded_rows(n)), dtype=torch.uint8, device=dev)
+    cols[:, :n] = rows.t()
+    want_l, got_l = (torch.empty((12, n), dtype=torch.int32, device=dev) for _ in range(2))
+    want = cf.predict(cols, n, 0.5, leaves=want_l)
+    for x in (rows, rows.contiguous(), rows.t().contiguous().t(), rows.long(), rows.cpu()):
+        assert torch.equal(_forest_predict(cf, x, None, 24, dev, 0.5, got_l), want) and torch.equal(got_l, want_l)
+    cf.close()

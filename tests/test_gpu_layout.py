@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,F", [(1, 1), (15, 16), (16, 17), (255, 127), (256, 128), (257, 129), (1000, 2376),
-                                 (4099, 31)])
+                                 (4099, 31), (4099, 32), ((1 << 20) - 5, 9), ((1 << 20) + 5, 6),
+                                 ((1 << 20) + 5, 7), ((1 << 20) + 5, 15), ((1 << 20) + 5, 16)])
 @pytest.mark.parametrize("gather", [False, True])
 def test_transpose_bins(hip, n, F, gather):
     import torch
@@ -23,9 +24,13 @@ def test_transpose_bins(hip, n, F, gather):
     perm = rng.permutation(n) if gather else None
     want = (X if perm is None else X[torch.from_numpy(perm).cuda()]).t()
     for src in (X, X.contiguous(), X.view(torch.int8), X.t().contiguous().t(), X.cpu().numpy()):
-        got = column_major_bins(src, perm, torch.device("cuda:0"), chunk_rows=512, limit=200)
+        chunk = 512 if n < 10_000 else 1 << 18
+        got = column_major_bins(src, perm, torch.device("cuda:0"), chunk_rows=chunk, limit=200)
         assert got.shape == (F, padded_rows(n))
         assert torch.equal(got[:, :n], want) and not bool(got[:, n:].any())
+        if int(want.max()):
+            with pytest.raises(ValueError, match="max_bins"):
+                column_major_bins(src, perm, torch.device("cuda:0"), chunk_rows=chunk, limit=int(want.max()))
 
 
 @pytest.mark.parametrize("limit", [1, 5, 127, 128, 129, 200, 255])
