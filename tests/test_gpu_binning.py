@@ -96,11 +96,13 @@ def test_device_binning_matches_reference_golden(hip):
 
 
 @pytest.mark.parametrize("n,f,nb", [(1, 1, 2), (127, 31, 3), (128, 32, 4), (129, 33, 17), (1000, 70, 129),
-                                    (5001, 5, 255), (300_000, 40, 64)])
+                                    (5001, 5, 255), (300_000, 40, 64), (399_999, 1, 5), (400_001, 1, 5),
+                                    (800_003, 2, 64), (300_001, 7, 128), (300_001, 7, 129), (300_001, 8, 255)])
 def test_bin_rows_shapes(hip, n, f, nb):
-    """Tile, feature-group and search-depth edges, strided and feature-major inputs, with and
-    without a row gather: bins equal NumPy's searchsorted (values on the edges, signed zeros,
-    infinities and NaN included), padding rows 0."""
+    """Tile, feature-group and search-depth edges, few features on either side of the counts that go
+    through a feature-major copy, strided and feature-major inputs, with and without a row gather:
+    bins equal NumPy's searchsorted (values on the edges, signed zeros, infinities and NaN included),
+    padding rows 0."""
     import torch
 
     from packboost_amd.data import apply_bins_device
