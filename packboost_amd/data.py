@@ -17,6 +17,7 @@ and +0.0, which a sort may leave in any order).
 
 from __future__ import annotations
 
+import warnings
 from dataclasses import dataclass
 from typing import Iterable, Sequence
 
@@ -162,7 +163,11 @@ def _float_matrix_device(X, device):
     Xn = np.asarray(ensure_numpy(X), dtype=np.float32)
     if not (Xn.flags.c_contiguous or Xn.flags.f_contiguous):
         Xn = np.ascontiguousarray(Xn)
-    return torch.from_numpy(Xn).to(device)
+    if Xn.flags.writeable:
+        return torch.from_numpy(Xn).to(device)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", UserWarning)  # of an array that is not writable: it is only read
+        return torch.from_numpy(Xn).to(device)
 
 
 def _few_features(n: int, F: int, num_edges: int) -> bool:

@@ -56,6 +56,22 @@ def test_tree_records():
         _tree_records(swapped)
 
 
+@pytest.mark.parametrize("order", ["C", "F"])
+def test_read_only_float_table(order):
+    """A read-only float table (a DataFrame's values can be one) reaches the device without a copy on the
+    host and without a warning; in a process of its own, since torch warns once."""
+    code = f"""
+import numpy as np, torch
+from packboost_amd.data import _float_matrix_device
+X = np.asarray(np.arange(12, dtype=np.float32).reshape(4, 3), order={order!r})
+X.flags.writeable = False
+x = _float_matrix_device(X, torch.device("cpu"))
+assert x.data_ptr() == X.ctypes.data and np.array_equal(x.numpy(), X)
+"""
+    run = subprocess.run([sys.executable, "-W", "error::UserWarning", "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert run.returncode == 0, run.stderr
+
+
 def test_subset_size_rule():
     from packboost_amd import PackBoostConfig
     from packboost_amd.engine import subset_size
