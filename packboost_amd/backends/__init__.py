@@ -54,7 +54,10 @@ def _u8_fm(bins: torch.Tensor) -> tuple[torch.Tensor, int]:
     if bins.dim() != 2:
         raise ValueError("bins must be 2-D feature-major [F, N]")
     N = int(bins.shape[1])
-    b = bins.view(torch.uint8) if bins.dtype == torch.int8 else bins.to(torch.uint8)
+    if bins.dtype == torch.uint8:
+        b = bins
+    else:
+        b = bins.view(torch.uint8) if bins.dtype == torch.int8 else bins.to(torch.uint8)
     if (N > 1 and b.stride(1) != 1) or b.stride(0) < N:
         b = b.contiguous()
     return b, max(int(b.stride(0)), N)
