@@ -97,9 +97,11 @@ __device__ __forceinline__ uint32_t order_key(float x) {
 // contiguous bytes of a row) and runs its 16 searches side by side, STEPS branchless LDS probes
 // each, so the probes' latencies overlap; the bins leave through LDS as 128-byte runs per column.
 // An odd stride between the features' edges keeps the first probes (the same index in every
-// feature) on distinct banks; the later ones are random. The LDS probes bound it
-// (a random one takes about 9 clocks): 1M x 500 values through 254 edges take 1.13 ms (440 G
-// values/s; 0.65 ms through 15 edges), where transposed copies and one search per lane took 9.0 ms.
+// feature) on distinct banks; the later ones are random. The LDS probes bound it (8.7 clocks each, three
+// quarters of them bank conflicts; the LDS is active 78% of the time): 1M x 500 values through 254 edges
+// take 1.13 to 1.17 ms (430 G values/s; 0.65 ms through 15 edges), where transposed copies and one search
+// per lane took 9.0 ms. The 32 features are searched however few there are: long tables of up to 7 are
+// binned column by column instead.
 // Edges that do not ascend (a column with infinities between its quantiles has NaN edges below
 // finite ones) take searchsorted's own probe order instead, which decides what it finds there.
 // All feature groups of a row range run on one XCD, where its rows' split cache lines are shared.

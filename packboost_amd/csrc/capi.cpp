@@ -422,7 +422,7 @@ int hist_build(pb_ctx* c, const uint8_t* bins, int64_t ld_bytes, int32_t nibble,
     groups = std::min<int64_t>(groups, need);
     // Enough workgroups to cover the chip: narrower tiles while a narrow frontier leaves fewer than
     // 1024 items (200k rows x 100 features x 128 bins in 50 eras, depths 0-1: 4-feature tiles 19.6 /
-    // 20.1 us against 26.6 / 22.4 for the widest that fit), a wider one fewer than one per CU (10k
+    // 20.1 us against 26.6 / 22.4 for the widest that fit), a wider one fewer than 256, one per CU (10k
     // rows x 20 features, depth 3: 8.4 against 10.3; at 416 items of 16 nodes a further halving lost,
     // 25.4 against 22.6 us: every tile re-reads the rows' state). Up to two nodes, where a part's flush is
     // short, eras that are all split go in finer parts too (one era of 200k rows x 64 features,

@@ -331,8 +331,9 @@ __device__ __forceinline__ uint32_t squeeze4(uint32_t x) {
 // LDS as raw bytes, `raw` (the tree block's space, unused until the walk), with an odd row stride
 // in dwords: a lane then reads the bytes of its own row and writes whole tile words, both free of
 // bank conflicts. 240 bytes are whole words at every packing (24, 30 or 60). 5M x 2376 codes
-// through 250 trees of depth 6: 3.1 ms (3.8 TB/s of rows read), where the column-major walk takes
-// 2.9 ms after 5.2 ms of transposition.
+// through 250 trees of depth 6: 3.1 to 3.7 ms box to box (3.2 to 3.8 TB/s of rows read), where the
+// column-major walk takes 2.9 to 3.4 ms after 5.2 ms of transposition. Fewer than 16 features leave the
+// 16-byte loads nearly empty: long tables of them take the column-major walk.
 template <int BITS, int NT, int R>
 __device__ __forceinline__ void stage_rows(const uint8_t* __restrict__ rows, int64_t N, int64_t stride, int F,
                                            const ForestTile& ft, int64_t r0, uint32_t* tile, uint32_t* raw) {

@@ -15,8 +15,8 @@
 //   select   a workgroup per quantile picks its ranks from its interval by radix selection, at any
 //            interval size, and interpolates in NumPy's order of operations
 // Columns of at most kSmall rows are sorted in LDS instead. Every step is exact; only speed depends
-// on the sample. 1M x 500 values and 254 quantiles take 6.9 ms (keys 1.0, count 3.1, gather 1.8,
-// select 0.9), where transposed copies, a segmented sort and its reading took 127 ms;
+// on the sample. 1M x 500 values and 254 quantiles take 6.6 ms (keys 0.9, count 2.5, gather 1.8,
+// select 1.2), where transposed copies, a segmented sort and its reading took 127 ms;
 // 200k x 100 and 127 quantiles 0.4 ms for 4.8.
 #include <algorithm>
 
@@ -184,7 +184,8 @@ __global__ __launch_bounds__(kSortBlock) void sample_kernel(Select st) {
     if (threadIdx.x == 0) st.nan[blockIdx.x] = 0u;
 }
 
-// Bound by the LDS probes (STEPS + 1 per key, mostly random); 8 searches per thread run side by side.
+// Bound by the LDS probes (STEPS + 1 per key, mostly random: 16 clocks each at STEPS 10, the LDS active
+// 95% of the time); 8 searches per thread run side by side.
 template <int STEPS>
 __global__ __launch_bounds__(kBlock) void count_kernel(Select st) {
     constexpr int kSplits = (1 << STEPS) - 1, kClasses = 2 << STEPS, kPer = 8;

@@ -468,9 +468,10 @@ bool pick_by_lane(int64_t MK, int32_t T) {
 // What a call's inputs must satisfy, looked up in one launch (RowlistFacts, cleared by the caller):
 // the first `wblocks` workgroups cover the weights and row counts, one (node, era) pair a thread up
 // to 512 workgroups (a single workgroup waited on its loads pair after pair: split search over
-// 1024 x 574 lists and 8 features 2.25 ms, 1.10 so), the others hess and the drawn columns' bins. The least and greatest weight - rows are joined as the
-// bit patterns of non-negative doubles, whose order is the numbers'; the least as its complement, so
-// that a cleared record is the neutral one of both.
+// 1024 x 574 lists and 8 features 2.25 ms, 1.10 so), the others hess and the drawn columns' bins.
+// The least and greatest weight - rows are joined as the bit patterns of non-negative doubles, whose
+// order is the numbers'; the least as its complement, so that a cleared record is the neutral one
+// of both.
 __global__ __launch_bounds__(kRlBlock) void rl_facts_kernel(
     const uint8_t* __restrict__ bins, int64_t N, int64_t ld, int32_t F, const int32_t* __restrict__ feats, int32_t K,
     const float* __restrict__ hess, int64_t n_hess, const float* __restrict__ weights, const int32_t* __restrict__ nes,
